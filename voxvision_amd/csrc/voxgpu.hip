@@ -21,7 +21,8 @@
 //
 // Floating point: compiled with -ffp-contract=off; __builtin_fmaf marks the
 // reference's fused sites (geom-sse.c:109,135; simple-camera.c:29;
-// vect-ops-sse.c:24).  Division is IEEE correctly rounded (HIP default).
+// vect-ops-sse.c:24).  Division is IEEE correctly rounded (HIP default), or
+// three operations that give the same bits (raymath.h).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -42,6 +43,7 @@
 #include "cull.h"
 #include "fastdiv.h"
 #include "lights.h"
+#include "raymath.h"
 #include "tree_build.h"
 #include "voxg_internal.h"
 #include "../../include/voxgpu_testing.h"
@@ -209,9 +211,9 @@ __device__ __forceinline__ float abs_metric(f3 a, f3 b) {
 
 // geom-sse.c:70-82
 __device__ __forceinline__ int corrected_subspace(f3 c, f3 p, f3 d) {
-    int bx = (p.x == c.x) ? (d.x < 0.0f) : (p.x < c.x);
-    int by = (p.y == c.y) ? (d.y < 0.0f) : (p.y < c.y);
-    int bz = (p.z == c.z) ? (d.z < 0.0f) : (p.z < c.z);
+    const int bx = (p.x < c.x) | ((p.x == c.x) & (d.x < 0.0f));
+    const int by = (p.y < c.y) | ((p.y == c.y) & (d.y < 0.0f));
+    const int bz = (p.z < c.z) | ((p.z == c.z) & (d.z < 0.0f));
     return bx | (by << 1) | (bz << 2);
 }
 
@@ -228,11 +230,52 @@ __device__ __forceinline__ bool box_ball(f3 bmin, f3 bmax, f3 c, float rr) {
     return ((dx + dy) + dz) < rr;
 }
 
+// A ray's direction with its reciprocals, for the tests of raymath.h; `odd`
+// (a ray or tree that is not plain) sends every test to the exact ones.
+struct Dir {
+    f3 d, y;
+    bool odd;
+};
+
+__device__ __forceinline__ Dir make_dir(f3 o, f3 d, uint32_t tree_odd) {
+    Dir r;
+    r.d = d;
+    r.y = f3{raymath::reciprocal(d.x), raymath::reciprocal(d.y),
+             raymath::reciprocal(d.z)};
+    const bool plain = raymath::plain_axis(o.x, d.x) &
+                       raymath::plain_axis(o.y, d.y) &
+                       raymath::plain_axis(o.z, d.z) &
+                       ((d.x != 0.0f) | (d.y != 0.0f) | (d.z != 0.0f));
+    r.odd = (tree_odd != 0) | !plain;
+    return r;
+}
+
+// hit_box by raymath::box_entry, by the exact test where that is undecided.
+// What bounds the traversal is VALU issue; with these tests and the
+// branch-free crossings() below, 16 M incoherent rays through the 256^3 CT
+// scene took 1.02e9 instead of 1.52e9 VALU instructions and the kernel
+// 2.28 -> 1.88 ms, 64 1080p BEST frames of it (one and a half diagonals of
+// the voxels' box away) 3.85 -> 3.13 ms.
+__device__ __forceinline__ bool hit_box_dir(f3 bmin, f3 bmax, f3 o,
+                                            const Dir &r, f3 &e) {
+    const float lo[3] = {bmin.x, bmin.y, bmin.z}, hi[3] = {bmax.x, bmax.y, bmax.z};
+    const float oo[3] = {o.x, o.y, o.z}, dd[3] = {r.d.x, r.d.y, r.d.z};
+    const float yy[3] = {r.y.x, r.y.y, r.y.z};
+    float ee[3];
+    const raymath::Verdict v = raymath::box_entry(lo, hi, oo, dd, yy, ee);
+    e = f3{ee[0], ee[1], ee[2]};
+    bool in = v == raymath::kHit;
+    if (__builtin_expect(r.odd | (v == raymath::kUndecided), 0))
+        in = hit_box(bmin, bmax, o, r.d, e);
+    return in;
+}
+
 struct Tree {
     const NodeRec *__restrict__ nodes;
     const float *__restrict__ dots;
     float vx, vy, vz;
-    uint32_t empty;
+    uint16_t empty;
+    uint16_t odd;  // not plain (raymath.h): the exact tests only
     float ivx, ivy, ivz;  // 1/V when V is a power of two, else 0
     uint32_t ncut;        // boxes of the render pre-pass's cut (0: none)
     const float *__restrict__ cut;  // 6 floats per box: min, max
@@ -284,9 +327,78 @@ __device__ __forceinline__ uint32_t dense_voxel(const Node &n, f3 r,
     return n.ref + (uint32_t)((ix * dy + iy) * dz + iz);
 }
 
-__device__ __forceinline__ uint32_t child_of(uint32_t ref, uint32_t mask,
-                                             int s) {
-    return ((mask >> s) & 1u) ? ref + __popc(mask & ((1u << s) - 1u)) : kEnd;
+// What an inner node's entry point decides (search.c:84-134): the subspace
+// it lies in and the dividing planes that the ray hits inside the node's
+// box, nearest first by L1 distance from the entry, as axis bits (0: none
+// further).
+struct Cross {
+    uint32_t s, b1, b2, b3;
+};
+
+// The reference's steps one by one: compaction of the hits in plane order
+// (:108-113), then a selection sort by swaps (:115-134).  Both are one
+// network over (distance, axis bit) in which a plane that is not hit comes
+// after any that is.
+__device__ __forceinline__ Cross crossings_exact(const Node &nd, f3 e, f3 d) {
+    f3 P0 = e, P1 = e, P2 = e;
+    const bool h0 = hit_plane(e, d, nd.c, 0, nd.bmin, nd.bmax, P0);
+    const bool h1 = hit_plane(e, d, nd.c, 1, nd.bmin, nd.bmax, P1);
+    const bool h2 = hit_plane(e, d, nd.c, 2, nd.bmin, nd.bmax, P2);
+    const float m0 = abs_metric(e, P0), m1 = abs_metric(e, P1),
+                m2 = abs_metric(e, P2);
+    const bool sa = h1 && (!h0 || m1 < m0);  // swap 0, 1
+    const float lo_m = sa ? m1 : m0, hi_m = sa ? m0 : m1;
+    const bool lo_v = h0 || h1, hi_v = h0 && h1;
+    const uint32_t lo_b = !lo_v ? 0u : sa ? 2u : 1u;
+    const uint32_t hi_b = !hi_v ? 0u : sa ? 1u : 2u;
+    const bool sb = h2 && (!lo_v || m2 < lo_m);  // swap 0, 2
+    const float z_m = sb ? lo_m : m2;
+    const uint32_t b2 = h2 ? 4u : 0u, z_b = sb ? lo_b : b2;
+    const bool sc = z_b && (!hi_v || z_m < hi_m);  // swap 1, 2
+    Cross x;
+    x.s = (uint32_t)corrected_subspace(nd.c, e, d);
+    x.b1 = sb ? b2 : lo_b;
+    x.b2 = sc ? z_b : hi_b;
+    x.b3 = sc ? hi_b : z_b;
+    return x;
+}
+
+// The same by raymath::plane_point, for a plain ray: the distances are then
+// finite, so an infinite one stands for a plane that is not hit.
+__device__ __forceinline__ Cross crossings(const Node &nd, f3 e, const Dir &r) {
+    const float lo[3] = {nd.bmin.x, nd.bmin.y, nd.bmin.z};
+    const float hi[3] = {nd.bmax.x, nd.bmax.y, nd.bmax.z};
+    const float ee[3] = {e.x, e.y, e.z}, dd[3] = {r.d.x, r.d.y, r.d.z};
+    const float yy[3] = {r.y.x, r.y.y, r.y.z}, c[3] = {nd.c.x, nd.c.y, nd.c.z};
+    float m[3];
+    uint32_t b[3], key[3], s = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        float p[3], a;
+        const bool h = raymath::plane_point(lo, hi, ee, dd, yy, c[i], i, a, p);
+        m[i] = h ? abs_metric(e, f3{p[0], p[1], p[2]}) : INFINITY;
+        b[i] = h ? 1u << i : 0u;
+        key[i] = raymath::size_key(a);
+        // corrected_subspace: e below c, or on it and d negative (y has
+        // d's sign, and is +0 for a zero)
+        s |= (raymath::bits(a == 0.0f ? yy[i] : -a) >> 31) << i;
+    }
+    const bool sa = m[1] < m[0];
+    const float lo_m = sa ? m[1] : m[0], hi_m = sa ? m[0] : m[1];
+    const uint32_t lo_b = sa ? b[1] : b[0], hi_b = lo_b ^ b[0] ^ b[1];
+    const bool sb = m[2] < lo_m;
+    const float z_m = sb ? lo_m : m[2];
+    const bool sc = z_m < hi_m;
+    Cross x;
+    x.s = s;
+    x.b1 = sb ? b[2] : lo_b;
+    const uint32_t z_b = x.b1 ^ lo_b ^ b[2];
+    x.b2 = sc ? z_b : hi_b;
+    x.b3 = x.b2 ^ z_b ^ hi_b;
+    if (__builtin_expect(r.odd | (raymath::min3(key[0], key[1], key[2]) <
+                                  raymath::kTinyKey), 0))
+        x = crossings_exact(nd, e, r.d);
+    return x;
 }
 
 __device__ __forceinline__ uint32_t lane_id() {
@@ -469,9 +581,8 @@ constexpr size_t kCounterBytes =
 // waiting for a wave-wide refill.
 template <class Src, class Sink>
 struct ChunkWork {
-    // no occupancy floor asked of the register allocator (it fits 7 waves
-    // per SIMD as it is; 8 would spill)
-    static constexpr int kMinWavesPerSimd = 1;
+    // 8 waves per SIMD (at most 64 VGPRs; it takes 54)
+    static constexpr int kMinWavesPerSimd = 8;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return false; }
     // XCD hand-out: one contiguous range of the units per XCD
     __device__ __forceinline__ uint32_t xcd_group() const { return 0; }
@@ -517,8 +628,7 @@ struct BatchItem {
 // traverses that item's tree.
 template <class Src, class Sink>
 struct MultiWork {
-    // 6 waves per SIMD (at most 80 VGPRs) fit without spilling
-    static constexpr int kMinWavesPerSimd = 6;
+    static constexpr int kMinWavesPerSimd = 8;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return false; }
     __device__ __forceinline__ uint32_t xcd_group() const { return 0; }
     __device__ __forceinline__ uint32_t unit_shift() const { return 0; }
@@ -528,8 +638,7 @@ struct MultiWork {
     uint32_t n_items, chunk;
     __device__ __forceinline__ uint32_t prepare(uint32_t n) { return n; }
     struct State {
-        uint32_t ray, end;
-        Tree t;
+        uint32_t ray, end, item;
     };
     __device__ __forceinline__ void begin(uint32_t unit, State &st,
                                           uint32_t &cur, f3 &org, f3 &d) const {
@@ -540,7 +649,7 @@ struct MultiWork {
             else hi = mid - 1;
         }
         const BatchItem &it = items[lo];
-        st.t = it.t;
+        st.item = lo;
         st.ray = it.ray_begin + (unit - it.unit_begin) * chunk;
         st.end = min(st.ray + chunk, it.ray_begin + it.ray_count);
         src.get(st.ray, org, d);
@@ -558,7 +667,7 @@ struct MultiWork {
     __device__ __forceinline__ void flush(const State &, Ctrl *) const {}
     __device__ __forceinline__ const Tree &tree(const State &st,
                                                 const Tree &) const {
-        return st.t;
+        return items[st.item].t;
     }
 };
 
@@ -583,7 +692,7 @@ __device__ __forceinline__ float sqr_metric(f3 a, f3 b) {
 // the search).  Writes the voxel id and the hit point; false: no voxel.
 template <bool COUNT, bool PREFETCH = false>
 __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
-                                            f3 e, f3 d, uint32_t &vid,
+                                            f3 e, const Dir &d, uint32_t &vid,
                                             f3 &bres,
                                             unsigned long long &nt) {
     bres = e;
@@ -617,7 +726,7 @@ __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
                 f3 vmax = f3{vmin.x + V.x, vmin.y + V.y, vmin.z + V.z};
                 f3 far;
                 if (COUNT) nt++;
-                if (hit_box(vmin, vmax, e, d, far)) {
+                if (hit_box_dir(vmin, vmax, e, d, far)) {
                     float m = abs_metric(e, far);
                     if (m == 0.0f) {
                         bres = far;
@@ -641,7 +750,7 @@ __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
         f3 vmax = f3{vmin.x + V.x, vmin.y + V.y, vmin.z + V.z};
         f3 far;
         if (COUNT) nt++;
-        if (hit_box(vmin, vmax, e, d, far)) {
+        if (hit_box_dir(vmin, vmax, e, d, far)) {
             float m = abs_metric(e, far);
             if (m == 0.0f) {
                 bres = far;
@@ -957,9 +1066,8 @@ struct SpecOut {
 template <int MODE>
 struct BestWorkT {
     static constexpr bool SETS = MODE == 2;
-    // 7 waves per SIMD (at most 72 VGPRs): the compiler fits this kernel
-    // without spilling, and the extra wave hides node-load latency
-    static constexpr int kMinWavesPerSimd = 7;
+    // 8 waves per SIMD (at most 64 VGPRs)
+    static constexpr int kMinWavesPerSimd = 8;
     RenderItem one;
     SpecOut spec;            // MODE 1, 2: the root searches, for
                              // resolve_kernel, instead of the job's outputs
@@ -1110,7 +1218,9 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
     bool active = false;
     bool exhausted = false;
     uint32_t cur = 0;
-    f3 d{0, 0, 0}, org{0, 0, 0};
+    f3 org{0, 0, 0};
+    Dir dir;
+    std::memset(&dir, 0, sizeof(dir));
     // lane phase: traversing, waiting at a leaf whose box it entered (entry
     // point in org), or ended with a result
     // in (p_hit, p_vid, cur, org) that waits to be handed to the work unit
@@ -1146,9 +1256,17 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                 const uint32_t my = base + lanes_below(idle);
                 const uint32_t u = ((my / xch) * kXcds + x) * xch + my % xch;
                 if (my < r_len && u < n) {
+                    f3 d;
                     work.begin(u, st, cur, org, d);
+                    const Tree &T = work.tree(st, t);
+                    dir = make_dir(org, d, T.odd);
                     sp = lo = 0;
                     ph = PH_TRAV;
+                    if (T.empty) {  // no node to visit: a miss
+                        ph = PH_DONE;
+                        p_hit = false;
+                        p_vid = kEnd;
+                    }
                     active = true;
                     if (COUNT) {
                         if (cur == 0) nr++;
@@ -1169,13 +1287,9 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         // phase 1: one node of every traversing lane (search.c:8-29, 84-148)
         if (ph == PH_TRAV) {
             f3 e = org;
-            Node nd;
-            bool in = false;
-            if (!T.empty) {
-                nd = load_node(T.nodes, cur);
-                if (COUNT) nv++;
-                in = hit_box(nd.bmin, nd.bmax, org, d, e);
-            }
+            const Node nd = load_node(T.nodes, cur);
+            if (COUNT) nv++;
+            const bool in = hit_box_dir(nd.bmin, nd.bmax, org, dir, e);
             if (!in) {
                 popme = true;
             } else if ((nd.info & NT_TYPE_MASK) != NT_INNER) {
@@ -1184,82 +1298,21 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                 org = e;
             } else {
                 // search.c:84-148
-                int s = corrected_subspace(nd.c, e, d);
-                f3 P0, P1, P2;
-                bool h0 = hit_plane(e, d, nd.c, 0, nd.bmin, nd.bmax, P0);
-                bool h1 = hit_plane(e, d, nd.c, 1, nd.bmin, nd.bmax, P1);
-                bool h2 = hit_plane(e, d, nd.c, 2, nd.bmin, nd.bmax, P2);
-                // compact the hits in plane order (:108-113)
-                int cntp = 0, i0 = 0, i1 = 0, i2 = 0;
-                f3 Q0 = P0, Q1 = P1, Q2 = P2;
-                if (h0) {
-                    i0 = 0;
-                    Q0 = P0;
-                    cntp = 1;
-                }
-                if (h1) {
-                    if (cntp == 0) {
-                        i0 = 1;
-                        Q0 = P1;
-                    } else {
-                        i1 = 1;
-                        Q1 = P1;
-                    }
-                    cntp++;
-                }
-                if (h2) {
-                    if (cntp == 0) {
-                        i0 = 2;
-                        Q0 = P2;
-                    } else if (cntp == 1) {
-                        i1 = 2;
-                        Q1 = P2;
-                    } else {
-                        i2 = 2;
-                        Q2 = P2;
-                    }
-                    cntp++;
-                }
-                // selection sort by L1 distance from the entry (:115-134)
-                float m0 = abs_metric(e, Q0), m1 = abs_metric(e, Q1),
-                      m2 = abs_metric(e, Q2);
-                if (cntp >= 2 && m1 < m0) {
-                    f3 tq = Q0; Q0 = Q1; Q1 = tq;
-                    int ti = i0; i0 = i1; i1 = ti;
-                    float tv = m0; m0 = m1; m1 = tv;
-                }
-                if (cntp >= 3 && m2 < m0) {
-                    f3 tq = Q0; Q0 = Q2; Q2 = tq;
-                    int ti = i0; i0 = i2; i2 = ti;
-                    float tv = m0; m0 = m2; m2 = tv;
-                }
-                if (cntp >= 3 && m2 < m1) {
-                    f3 tq = Q1; Q1 = Q2; Q2 = tq;
-                    int ti = i1; i1 = i2; i2 = ti;
-                }
-                uint32_t mask = (nd.info >> 8) & 0xffu;
-                int s1 = s ^ (1 << i0);
-                int s2 = s1 ^ (1 << i1);
-                int s3 = s2 ^ (1 << i2);
-                uint32_t cs0 = child_of(nd.ref, mask, s);
-                // the children behind the planes that exist, in visiting
-                // order (:137-147), as (plane, child offset) pairs of a
-                // pending list: count in bits 0-1, pair j in bits 2+5j..
-                uint32_t lst = 0u, np = 0u;
-                auto pend = [&](int sub, int plane) {
-                    if ((mask >> sub) & 1u) {
-                        const uint32_t off =
-                            (uint32_t)__popc(mask & ((1u << sub) - 1u));
-                        lst |= ((uint32_t)plane | (off << 2)) << (2u + 5u * np);
-                        np++;
-                    }
+                const Cross x = crossings(nd, e, dir);
+                // the children behind the planes in visiting order
+                // (:137-147), those that exist: a pending list of 6-bit
+                // (axis bit, subspace) entries, the next one in the low bits
+                const uint32_t mask = (nd.info >> 8) & 0xffu;
+                const uint32_t s = x.s, s1 = s ^ x.b1, s2 = s1 ^ x.b2, s3 = s2 ^ x.b3;
+                auto there = [&](uint32_t c, uint32_t b) {
+                    return (((mask >> c) & 1u) != 0) & (b != 0);
                 };
-                if (cntp >= 1) pend(s1, i0);
-                if (cntp >= 2) pend(s2, i1);
-                if (cntp >= 3) pend(s3, i2);
+                uint32_t lst = there(s3, x.b3) ? x.b3 | (s3 << 3) : 0u;
+                lst = there(s2, x.b2) ? (lst << 6) | (s2 << 3) | x.b2 : lst;
+                lst = there(s1, x.b1) ? (lst << 6) | (s1 << 3) | x.b1 : lst;
                 // one stack entry for the node: its index and entry point,
                 // the plane points are recomputed when the entry is popped
-                if (np) {
+                if (lst) {
                     if (sp - lo == K) {
                         // ring full: its oldest entry goes to the spill
                         // buffer (or is dropped past the bound: reported)
@@ -1278,11 +1331,11 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                     ring[ri] = make_uint4(cur, __float_as_uint(e.x),
                                           __float_as_uint(e.y),
                                           __float_as_uint(e.z));
-                    ring_st[ri] = lst | np;
+                    ring_st[ri] = lst;
                     sp++;
                 }
-                if (cs0 != kEnd) {
-                    cur = cs0;
+                if ((mask >> s) & 1u) {
+                    cur = nd.ref + __popc(mask & ((1u << s) - 1u));
                     org = e;
                 } else {
                     popme = true;
@@ -1298,7 +1351,7 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
             const Node nd = load_node(T.nodes, cur);
             uint32_t vid = kEnd;
             f3 bres = org;
-            const bool hit = leaf_search<COUNT>(T, nd, org, d, vid, bres, nt);
+            const bool hit = leaf_search<COUNT>(T, nd, org, dir, vid, bres, nt);
             if (hit) {
                 ph = PH_DONE;
                 p_hit = true;
@@ -1334,22 +1387,29 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                 const uint32_t ri = ((sp - 1) & (K - 1)) * bdim + tid;
                 const uint4 v = ring[ri];
                 const uint32_t lst = ring_st[ri];
-                const uint32_t np = lst & 3u, pair = (lst >> 2) & 31u;
-                if (np == 1u) sp--;
-                else ring_st[ri] = (np - 1u) | ((lst >> 5) & ~3u);
-                const int p = (int)(pair & 3u);
+                if (lst < 64u) sp--;
+                else ring_st[ri] = lst >> 6;
+                const uint32_t ax = lst & 7u, sub = (lst >> 3) & 7u;
                 const f3 e = f3{__uint_as_float(v.y), __uint_as_float(v.z),
                                 __uint_as_float(v.w)};
                 const uint32_t *rec =
                     reinterpret_cast<const uint32_t *>(T.nodes + v.x);
                 const uint32_t ref = rec[offsetof(NodeRec, ref) / 4];
+                const uint32_t mask = (rec[offsetof(NodeRec, info) / 4] >> 8) & 0xffu;
                 const float cp =
-                    __uint_as_float(rec[offsetof(NodeRec, c) / 4 + p]);
-                const float k = (cp - comp(e, p)) / comp(d, p);
-                org = f3{__builtin_fmaf(k, d.x, e.x),
-                         __builtin_fmaf(k, d.y, e.y),
-                         __builtin_fmaf(k, d.z, e.z)};
-                cur = ref + (pair >> 2);
+                    __uint_as_float(rec[offsetof(NodeRec, c) / 4 + (ax >> 1)]);
+                auto on_axis = [&](f3 a) {
+                    return ax == 1u ? a.x : (ax == 2u ? a.y : a.z);
+                };
+                const float a = cp - on_axis(e), dp = on_axis(dir.d);
+                float k = raymath::quotient(a, dp, on_axis(dir.y));
+                if (__builtin_expect(dir.odd | (raymath::size_key(a) <
+                                                raymath::kTinyKey), 0))
+                    k = a / dp;
+                org = f3{__builtin_fmaf(k, dir.d.x, e.x),
+                         __builtin_fmaf(k, dir.d.y, e.y),
+                         __builtin_fmaf(k, dir.d.z, e.z)};
+                cur = ref + __popc(mask & ((1u << sub) - 1u));
             }
             if (cur == kEnd) {
                 ph = PH_DONE;
@@ -1362,9 +1422,11 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         const uint64_t dm = __ballot(ph == PH_DONE);
         const uint64_t am = __ballot(true);
         if (ph == PH_DONE && ((uint32_t)__popcll(dm) >= fin_batch || dm == am)) {
-            ph = PH_TRAV;
+            ph = T.empty ? PH_DONE : PH_TRAV;  // (an empty tree: all miss)
             sp = lo = 0;
+            f3 d = dir.d;
             if (work.finish(st, p_hit, p_vid, cur, org, cur, org, d)) {
+                dir = make_dir(org, d, T.odd);
                 if (COUNT) {
                     if (cur == 0) nr++;
                     else nl++;
@@ -1896,9 +1958,10 @@ resolve_kernel(RenderItem it, SpecOut spec, const uint32_t *__restrict__ queue,
                             ln = load_node(T.nodes, leaf);
                             loaded = leaf;
                         }
+                        const Dir dr = make_dir(o, d, T.odd);
                         f3 e;
-                        if (hit_box(ln.bmin, ln.bmax, o, d, e) &&
-                            leaf_search<false, true>(T, ln, e, d, svid, spt, nt)) {
+                        if (hit_box_dir(ln.bmin, ln.bmax, o, dr, e) &&
+                            leaf_search<false, true>(T, ln, e, dr, svid, spt, nt)) {
                             st = true;
                             kept = true;  // the leaf stays the same
                         }
@@ -1941,10 +2004,11 @@ resolve_kernel(RenderItem it, SpecOut spec, const uint32_t *__restrict__ queue,
                     ln = load_node(T.nodes, leaf);
                     loaded = leaf;
                 }
+                const Dir dr = make_dir(o, d, T.odd);
                 f3 e, pt;
                 uint32_t vid = kEnd;
-                if (hit_box(ln.bmin, ln.bmax, o, d, e) &&
-                    leaf_search<false, true>(T, ln, e, d, vid, pt, nt)) {
+                if (hit_box_dir(ln.bmin, ln.bmax, o, dr, e) &&
+                    leaf_search<false, true>(T, ln, e, dr, vid, pt, nt)) {
                     store(p, vid, pt);
                     vid_last = vid;
                     inter_last = pt;
@@ -2272,6 +2336,7 @@ struct voxg_tree {
     float *d_dots = nullptr;
     float *d_cut = nullptr;
     uint32_t ncut = 0;
+    bool odd = false;  // not plain (raymath.h)
     void *d_mem = nullptr;
     size_t bytes = 0;
     int device = 0;
@@ -2316,10 +2381,10 @@ std::mutex g_mu;
 // finish_batch, split_best per kind of launch (fastest measured on the
 // 256^3 benchmark scene; every field is validated by voxg_set_*)
 voxg_launch_config g_cfg[VOXG_LAUNCH_KINDS] = {
-    {4, 256, 28, 8, 1, 1, 24, 16, 0},   // VOXG_LAUNCH_RAYS
+    {4, 256, 32, 8, 1, 1, 24, 20, 0},   // VOXG_LAUNCH_RAYS
     {4, 256, 24, 8, 4, 1, 16, 16, 0},   // VOXG_LAUNCH_RENDER
     {4, 256, 28, 48, 4, 1, 32, 64, 4},  // VOXG_LAUNCH_RENDER_BEST
-    {4, 256, 24, 8, 1, 1, 16, 16, 0},   // VOXG_LAUNCH_BATCH
+    {4, 256, 32, 8, 1, 1, 24, 32, 0},   // VOXG_LAUNCH_BATCH
 };
 
 voxg_launch_config current_config(int kind) {
@@ -2548,6 +2613,7 @@ dev::Tree dev_tree(const voxg_tree *t) {
     d.ivy = pow2_inverse(d.vy);
     d.ivz = pow2_inverse(d.vz);
     d.empty = t->host.nodes.empty() ? 1u : 0u;
+    d.odd = t->odd ? 1u : 0u;
     d.ncut = t->ncut;
     d.cut = t->d_cut;
     return d;
@@ -2711,8 +2777,26 @@ int upload(voxg_tree *t) {
     return 0;
 }
 
+// Whether the tests of raymath.h hold for the tree: its boxes, centres and
+// voxels finite, at most 2^60 in magnitude and not inverted.
+bool plain_tree(const HostTree &h) {
+    // (a count without branches, which the compiler vectorises)
+    size_t off = 0;
+    auto far = [](float x) { return (size_t)!(std::fabs(x) <= 0x1p60f); };
+    for (const NodeRec &n : h.nodes) {
+        for (int k = 0; k < 3; k++)
+            off += far(n.bmin[k]) + far(n.bmax[k]) +
+                   (size_t)!(n.bmin[k] <= n.bmax[k]);
+        if (node_type(n.info) == NT_INNER)
+            off += far(n.c[0]) + far(n.c[1]) + far(n.c[2]);
+    }
+    for (float x : h.dots) off += far(x);
+    return off + far(h.voxel[0]) + far(h.voxel[1]) + far(h.voxel[2]) == 0;
+}
+
 int finish_tree(voxg_tree *t, voxg_tree **out) {
     t->stack_bound = stack_bound_of(t->host);
+    t->odd = !plain_tree(t->host);
     int rc = upload(t);
     if (rc) {
         if (t->d_mem) (void)hipFree(t->d_mem);
