@@ -155,6 +155,14 @@ struct f3 {
     float x, y, z;
 };
 
+// p as a pointer to device memory: the compiler cannot tell for a pointer
+// that it loads from memory itself, and would access it through the flat
+// path, which also waits for LDS.
+template <class T>
+__device__ __forceinline__ T *global(T *p) {
+    return (T *)(__attribute__((address_space(1))) T *)p;
+}
+
 // geom-sse.c:84-116 (fit_into_box :34-40)
 __device__ __forceinline__ bool hit_box(f3 bmin, f3 bmax, f3 o, f3 d, f3 &r) {
     float fx = smin(smax(o.x, bmin.x), bmax.x);
@@ -294,7 +302,7 @@ struct Node {
 
 __device__ __forceinline__ Node load_node(const NodeRec *__restrict__ nodes,
                                           uint32_t i) {
-    const float4 *p = reinterpret_cast<const float4 *>(nodes + i);
+    const float4 *p = global(reinterpret_cast<const float4 *>(nodes + i));
     float4 a = p[0], b = p[1], c = p[2];
     Node n;
     n.bmin = f3{a.x, a.y, a.z};
@@ -417,8 +425,8 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
 struct SoaSrc {
     const float *ox, *oy, *oz, *dx, *dy, *dz;
     __device__ __forceinline__ void get(uint32_t r, f3 &o, f3 &d) const {
-        o = f3{ox[r], oy[r], oz[r]};
-        d = f3{dx[r], dy[r], dz[r]};
+        o = f3{global(ox)[r], global(oy)[r], global(oz)[r]};
+        d = f3{global(dx)[r], global(dy)[r], global(dz)[r]};
     }
 };
 
@@ -427,12 +435,12 @@ struct SoaSink {
     float *hx, *hy, *hz;
     __device__ __forceinline__ void put(uint32_t r, bool hit, uint32_t vid,
                                         uint32_t leafi, f3 p) const {
-        if (voxel) voxel[r] = hit ? vid : kEnd;
-        if (leaf) leaf[r] = hit ? leafi : kEnd;
+        if (voxel) global(voxel)[r] = hit ? vid : kEnd;
+        if (leaf) global(leaf)[r] = hit ? leafi : kEnd;
         if (hit && hx) {
-            hx[r] = p.x;
-            hy[r] = p.y;
-            hz[r] = p.z;
+            global(hx)[r] = p.x;
+            global(hy)[r] = p.y;
+            global(hz)[r] = p.z;
         }
     }
 };
@@ -486,7 +494,7 @@ struct Shade {
         L[2] = amb[2];
         uint32_t n = 0;
         while (n < nlnodes) {
-            const LightNode nd = lnodes[n];
+            const LightNode nd = global(lnodes)[n];
             if (!(dist2(nd.c, p) < nd.sqr_radius)) {
                 n = nd.escape;
                 continue;
@@ -497,7 +505,7 @@ struct Shade {
             }
             const uint32_t cnt = nd.info >> 8;
             for (uint32_t k = 0; k < cnt; k++) {
-                const LightRec sp = lsph[nd.first + k];
+                const LightRec sp = global(lsph)[nd.first + k];
                 if (cnt == 1u || dist2(sp.c, p) < sp.sqr_radius) {
                     const float d = fminf(sp.radius, sqrtf(dist2(sp.c, p)));
                     const float a = 1.0f - d / sp.radius;
@@ -515,7 +523,7 @@ struct Shade {
         int x = abs((int)div_v(p.x, vx, ivx)) & 31;
         int y = abs((int)div_v(p.y, vy, ivy)) & 31;
         int z = abs((int)div_v(p.z, vz, ivz)) & 31;
-        uint32_t c = tex[x * 1024 + y * 32 + z];
+        uint32_t c = global(tex)[x * 1024 + y * 32 + z];
         if (!lnodes) return (c << rshift) | (c << gshift) | (c << bshift) | amask;
         float L[3];
         light(p, L);
@@ -534,21 +542,22 @@ struct PixSink {
     Shade sh;
     __device__ __forceinline__ void put(uint32_t r, bool hit, uint32_t vid,
                                         uint32_t, f3 p) const {
-        if (voxel) voxel[r] = hit ? vid : kEnd;
+        if (voxel) global(voxel)[r] = hit ? vid : kEnd;
         if (hit) {
             if (this->hit) {
-                this->hit[r] = p.x;
-                this->hit[plane + r] = p.y;
-                this->hit[2 * plane + r] = p.z;
+                float *const h = global(this->hit);
+                h[r] = p.x;
+                h[plane + r] = p.y;
+                h[2 * plane + r] = p.z;
             }
-            if (squares) squares[r] = sh.color(p);
+            if (squares) global(squares)[r] = sh.color(p);
         }
     }
 };
 
 struct Ctrl {
     uint32_t rdone;    // workgroups of resolve_kernel that have finished
-    uint32_t left;     // waves that have finished
+    uint32_t left;     // ranges (XCDs) whose waves have all finished
     uint32_t pad0;
     uint32_t pad;
     unsigned long long visits, tests, rays, leaf_trav;
@@ -583,18 +592,20 @@ template <class Src, class Sink>
 struct ChunkWork {
     // 8 waves per SIMD (at most 64 VGPRs; it takes 54)
     static constexpr int kMinWavesPerSimd = 8;
-    __host__ __device__ __forceinline__ bool keeps_queue() const { return false; }
+    static constexpr uint32_t kPool = 4, kFew = 0;
+    __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
     // XCD hand-out: one contiguous range of the units per XCD
-    __device__ __forceinline__ uint32_t xcd_group() const { return 0; }
-    __device__ __forceinline__ uint32_t unit_shift() const { return 0; }
-    Src src;
+    __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
+        Src src;
     Sink sink;
     uint32_t n, chunk;
-    __device__ __forceinline__ uint32_t prepare(uint32_t n) { return n; }
+    __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &) const {
+        return n;
+    }
     struct State {
         uint32_t ray, end;
     };
-    __device__ __forceinline__ void begin(uint32_t unit, State &st,
+    __device__ __forceinline__ void begin(uint32_t unit, uint32_t, State &st,
                                           uint32_t &cur, f3 &org, f3 &d) const {
         st.ray = unit * chunk;
         st.end = min(st.ray + chunk, n);
@@ -615,6 +626,10 @@ struct ChunkWork {
                                                 const Tree &t) const {
         return t;
     }
+    static __device__ __forceinline__ const NodeRec *nodes(const State &,
+                                                           const NodeRec *t) {
+        return t;
+    }
 };
 
 // One item of a multi-tree batch: a tree and a run of rays of the batch.
@@ -629,27 +644,31 @@ struct BatchItem {
 template <class Src, class Sink>
 struct MultiWork {
     static constexpr int kMinWavesPerSimd = 8;
-    __host__ __device__ __forceinline__ bool keeps_queue() const { return false; }
-    __device__ __forceinline__ uint32_t xcd_group() const { return 0; }
-    __device__ __forceinline__ uint32_t unit_shift() const { return 0; }
-    Src src;
+    static constexpr uint32_t kPool = 4, kFew = 0;
+    __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
+    __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
+        Src src;
     Sink sink;
     const BatchItem *items;
     uint32_t n_items, chunk;
-    __device__ __forceinline__ uint32_t prepare(uint32_t n) { return n; }
+    __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &) const {
+        return n;
+    }
     struct State {
         uint32_t ray, end, item;
+        const NodeRec *nodes;  // of the item's tree
     };
-    __device__ __forceinline__ void begin(uint32_t unit, State &st,
+    __device__ __forceinline__ void begin(uint32_t unit, uint32_t, State &st,
                                           uint32_t &cur, f3 &org, f3 &d) const {
         uint32_t lo = 0, hi = n_items - 1;
         while (lo < hi) {
             uint32_t mid = (lo + hi + 1) >> 1;
-            if (items[mid].unit_begin <= unit) lo = mid;
+            if (global(items)[mid].unit_begin <= unit) lo = mid;
             else hi = mid - 1;
         }
-        const BatchItem &it = items[lo];
+        const BatchItem &it = global(items)[lo];
         st.item = lo;
+        st.nodes = it.t.nodes;
         st.ray = it.ray_begin + (unit - it.unit_begin) * chunk;
         st.end = min(st.ray + chunk, it.ray_begin + it.ray_count);
         src.get(st.ray, org, d);
@@ -667,7 +686,11 @@ struct MultiWork {
     __device__ __forceinline__ void flush(const State &, Ctrl *) const {}
     __device__ __forceinline__ const Tree &tree(const State &st,
                                                 const Tree &) const {
-        return items[st.item].t;
+        return global(items)[st.item].t;
+    }
+    static __device__ __forceinline__ const NodeRec *nodes(const State &st,
+                                                           const NodeRec *) {
+        return st.nodes;
     }
 };
 
@@ -709,7 +732,7 @@ __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
         // the first 7 voxels' corners loaded together, not one round trip
         // per voxel
         float qx[7], qy[7], qz[7];
-        const float *base = T.dots + 3u * nd.ref;
+        const float *base = global(T.dots) + 3u * nd.ref;
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
             qx[k] = qy[k] = qz[k] = 0.0f;
@@ -745,7 +768,7 @@ __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
         k0 = 7;
     }
     for (uint32_t k = k0; k < cnt; k++) {
-        const float *p = T.dots + 3u * (nd.ref + k);
+        const float *p = global(T.dots) + 3u * (nd.ref + k);
         f3 vmin = f3{p[0], p[1], p[2]};
         f3 vmax = f3{vmin.x + V.x, vmin.y + V.y, vmin.z + V.z};
         f3 far;
@@ -801,32 +824,32 @@ struct BlockWork {
     // 6 waves per SIMD (at most 80 VGPRs) fit without spilling for one
     // render; the multi-job form would spill at that floor
     static constexpr int kMinWavesPerSimd = MULTI ? 1 : 6;
-    __host__ __device__ __forceinline__ bool keeps_queue() const { return false; }
+    static constexpr uint32_t kPool = 1, kFew = 0;
+    __host__ __device__ __forceinline__ bool keeps_queue() const { return MULTI; }
     // one render's block queue is ordered longest-first (block_cull_kernel)
     RenderItem one;             // the job when !MULTI
     const RenderItem *items;    // the jobs when MULTI, by unit_begin
     uint32_t n_items;
     const uint32_t *queue;      // !MULTI: units are queue entries if set:
     const unsigned long long *qpair;  // the first (low word) units from
-    uint32_t qlen;              // the front, the rest from the back of qlen
-    uint32_t qf;                // entries; qf: the low word, from prepare()
+    uint32_t qlen;              // the front (qf in begin(), from prepare()),
+                                // the rest from the back of qlen entries
     uint32_t group;             // !MULTI: units dealt to the XCDs in turns
-                                // of `group` (the queue is ordered
+                                // of 1 << group (the queue is ordered
                                 // longest-first, so every XCD should follow
                                 // that order); MULTI: contiguous ranges
-    __device__ __forceinline__ uint32_t xcd_group() const {
+    __device__ __forceinline__ uint32_t xcd_shift() const {
         if constexpr (MULTI) return 0;
         else return group;
     }
-    __device__ __forceinline__ uint32_t unit_shift() const { return 0; }
-    uint32_t units_per_block_host() const { return 1u; }
+        uint32_t units_per_block_host() const { return 1u; }
     // reads once per thread what the block pre-pass counted on the device;
     // returns the number of units
-    __device__ __forceinline__ uint32_t prepare(uint32_t n) {
+    __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &qf) const {
         if constexpr (!MULTI) {
             if (queue) {
                 uint32_t qt;
-                queue_counts(*qpair, qlen, qf, qt);
+                queue_counts(*global(qpair), qlen, qf, qt);
                 return qt;
             }
         }
@@ -835,6 +858,7 @@ struct BlockWork {
     enum { CORNER1 = 0, CORNER2 = 1, LOOP = 2 };
     struct State {
         uint32_t item, frame, base;  // job, frame in the job, output index
+        const NodeRec *nodes;        // MULTI: of the job's tree
         // packed in one word: the pixel position i in the block's order and
         // its end, the stage, the block's mode, ray merging, a leaf try
         uint32_t i : 5, iend : 5, stage : 2, mode : 2, merge : 1,
@@ -846,12 +870,12 @@ struct BlockWork {
     };
 
     __device__ __forceinline__ const RenderItem &item(const State &st) const {
-        if constexpr (MULTI) return items[st.item];
+        if constexpr (MULTI) return global(items)[st.item];
         else return one;
     }
     __device__ __forceinline__ const CamDev &cam(const State &st) const {
         const RenderItem &it = item(st);
-        return it.cams[st.frame];
+        return global(it.cams)[st.frame];
     }
     __device__ __forceinline__ void emit(const State &st, int p, bool hit,
                                          uint32_t vid, f3 e) const {
@@ -886,22 +910,24 @@ struct BlockWork {
         st.merged += st.merge ? 1u : 0u;
         return false;
     }
-    __device__ __forceinline__ void begin(uint32_t unit, State &st,
+    __device__ __forceinline__ void begin(uint32_t unit, uint32_t qf, State &st,
                                           uint32_t &cur, f3 &org, f3 &d) const {
         st.item = 0;
         if constexpr (!MULTI) {
-            if (queue) unit = queue[unit < qf ? unit : qlen - 1u - (unit - qf)];
+            if (queue)
+                unit = global(queue)[unit < qf ? unit : qlen - 1u - (unit - qf)];
         }
         if constexpr (MULTI) {
             uint32_t lo = 0, hi = n_items - 1;
             while (lo < hi) {
                 uint32_t mid = (lo + hi + 1) >> 1;
-                if (items[mid].unit_begin <= unit) lo = mid;
+                if (global(items)[mid].unit_begin <= unit) lo = mid;
                 else hi = mid - 1;
             }
             st.item = lo;
         }
         const RenderItem &it = item(st);
+        if constexpr (MULTI) st.nodes = it.t.nodes;
         uint32_t u = unit - it.unit_begin;
         // frames are stored one after the other in the square layout
         st.frame = it.bpf.div(u);
@@ -994,8 +1020,12 @@ struct BlockWork {
     }
     __device__ __forceinline__ const Tree &tree(const State &st,
                                                 const Tree &t) const {
-        if constexpr (MULTI) return items[st.item].t;
+        if constexpr (MULTI) return global(items)[st.item].t;
         else return t;
+    }
+    static __device__ __forceinline__ const NodeRec *nodes(const State &st,
+                                                           const NodeRec *t) {
+        return MULTI ? st.nodes : t;
     }
     __device__ __forceinline__ void flush(const State &st, Ctrl *ctrl) const {
         atomicAdd(&ctrl->fast_blocks, (unsigned long long)st.fast);
@@ -1024,12 +1054,12 @@ struct SpecOut {
     __device__ __forceinline__ void put(uint32_t blk, int px, bool hit,
                                         uint32_t v, uint32_t nd, f3 p) const {
         const uint32_t r = (uint32_t)px * stride + blk;
-        vid[r] = hit ? v : kEnd;
+        global(vid)[r] = hit ? v : kEnd;
         if (hit) {
-            node[r] = nd;
-            hx[r] = p.x;
-            hy[r] = p.y;
-            hz[r] = p.z;
+            global(node)[r] = nd;
+            global(hx)[r] = p.x;
+            global(hy)[r] = p.y;
+            global(hz)[r] = p.z;
         }
     }
     // direct FAST/ADAPTIVE renders: the leaf node of every pixel (kEnd on
@@ -1039,12 +1069,12 @@ struct SpecOut {
     // results themselves go to the outputs
     __device__ __forceinline__ void put_node(uint32_t blk, int px, bool hit,
                                              uint32_t nd, f3 p) const {
-        node[blk * 16u + (uint32_t)px] = hit ? nd : kEnd;
+        global(node)[blk * 16u + (uint32_t)px] = hit ? nd : kEnd;
         if (hit && (px == 0 || px == 15)) {
             const uint32_t c = (px == 15 ? stride : 0u) + blk;
-            cx[c] = p.x;
-            cy[c] = p.y;
-            cz[c] = p.z;
+            global(cx)[c] = p.x;
+            global(cy)[c] = p.y;
+            global(cz)[c] = p.z;
         }
     }
 };
@@ -1068,6 +1098,7 @@ struct BestWorkT {
     static constexpr bool SETS = MODE == 2;
     // 8 waves per SIMD (at most 64 VGPRs)
     static constexpr int kMinWavesPerSimd = 8;
+    static constexpr uint32_t kPool = 1, kFew = 8;
     RenderItem one;
     SpecOut spec;            // MODE 1, 2: the root searches, for
                              // resolve_kernel, instead of the job's outputs
@@ -1077,26 +1108,26 @@ struct BestWorkT {
     }
     const uint32_t *queue;  // block queue of the pre-pass, or null: the
     const unsigned long long *qpair;  // first (low word) entries from the
-    uint32_t qlen, qf;      // front, the rest from the back of qlen entries
+    uint32_t qlen;          // front (qf in begin(), from prepare()), the
+                            // rest from the back of qlen entries
     uint32_t split;         // a unit is 16 >> split pixels
-    uint32_t group;         // units dealt to the XCDs in turns of `group`
+    uint32_t group;         // units dealt to the XCDs in turns of 1 << group
     // SETS only: one pixel per unit of 1: pixels 0, 2, ..., 14 and 15 of
     // the block's order (9 units per block) or 2: pixels 1, 3, ..., 13 (7
     // units); pdiv divides by the units per block
     uint32_t pset;
     FastDiv pdiv;
-    __device__ __forceinline__ uint32_t xcd_group() const { return group; }
-    __device__ __forceinline__ uint32_t unit_shift() const { return split; }
+    __device__ __forceinline__ uint32_t xcd_shift() const { return group; }
     uint32_t units_per_block_host() const {
         if constexpr (SETS) return pdiv.d;
         else return 1u << split;
     }
     // reads once per thread what the block pre-pass counted on the device;
     // returns the number of units
-    __device__ __forceinline__ uint32_t prepare(uint32_t n) {
+    __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &qf) const {
         if (!queue) return n;
         uint32_t qt;
-        queue_counts(*qpair, qlen, qf, qt);
+        queue_counts(*global(qpair), qlen, qf, qt);
         if constexpr (SETS) return qt * pdiv.d;
         else return qt << split;
     }
@@ -1111,13 +1142,13 @@ struct BestWorkT {
     __device__ __forceinline__ void trace(const State &st, uint32_t &cur,
                                           f3 &org, f3 &d) const {
         const int p = render_order((int)(st.pos & 0xffu));
-        const CamDev &c = one.cams[st.frame];
+        const CamDev &c = global(one.cams)[st.frame];
         d = screen2world(c, (int)(st.xy & 0xffffu) + (p & 3),
                          (int)(st.xy >> 16) + (p >> 2));
         org = f3{c.px, c.py, c.pz};
         cur = 0;
     }
-    __device__ __forceinline__ void begin(uint32_t unit, State &st,
+    __device__ __forceinline__ void begin(uint32_t unit, uint32_t qf, State &st,
                                           uint32_t &cur, f3 &org, f3 &d) const {
         uint32_t b, i, len, own;
         if constexpr (SETS) {
@@ -1133,7 +1164,7 @@ struct BestWorkT {
             i = part * len;
             own = part == 0u;
         }
-        if (queue) b = queue[b < qf ? b : qlen - 1u - (b - qf)];
+        if (queue) b = global(queue)[b < qf ? b : qlen - 1u - (b - qf)];
         // frames are stored one after the other in the square layout
         st.frame = one.bpf.div(b);
         const uint32_t cs = b - st.frame * one.bpf.d;
@@ -1164,6 +1195,10 @@ struct BestWorkT {
                                                 const Tree &t) const {
         return t;
     }
+    static __device__ __forceinline__ const NodeRec *nodes(const State &,
+                                                           const NodeRec *t) {
+        return t;
+    }
     __device__ __forceinline__ void flush(const State &st, Ctrl *ctrl) const {
         atomicAdd(&ctrl->best_blocks, (unsigned long long)st.best);
     }
@@ -1178,43 +1213,138 @@ using BestDirectWork = BestWorkT<3>;
 // ---------------------------------------------------------------------------
 constexpr uint32_t kXcds = 8;        // XCDs of an MI355X
 constexpr uint32_t kXcdStride = 64;  // counters 256 bytes apart
+// The kernel's arguments, one struct at the start of the argument segment.
+template <class Work>
+struct TravArgs {
+    Tree t;
+    Work work;
+    uint32_t n;
+    Ctrl *ctrl;
+    uint32_t *ovf, *xnext;
+    uint4 *spill;
+    uint32_t spill_slots, width, refill, fin_batch, leaf_batch;
+};
+
+// The spill buffer's slot of stack entry i of a lane: entries
+// [spill_slots][lanes], then their pending lists; lanes numbered through
+// the grid, `width` a wave.
+struct SpillSlot {
+    uint4 *entry;
+    uint32_t *list;
+    template <class Args>
+    __device__ __forceinline__ SpillSlot(const Args &A, uint32_t wg_waves,
+                                         uint32_t wave, uint32_t lane, int i) {
+        const size_t lanes = (size_t)gridDim.x * wg_waves * A.width;
+        const size_t at = (size_t)i * lanes +
+                          (blockIdx.x * wg_waves + wave) * A.width + lane;
+        entry = global(A.spill) + at;
+        list = reinterpret_cast<uint32_t *>(global(A.spill) +
+                                            (size_t)A.spill_slots * lanes) + at;
+    }
+};
+
+// The arguments read from the argument segment when they are needed.  Used
+// as ordinary parameters the compiler loads them all before the loop, and
+// the sinks and cameras of a render do not fit the scalar registers of 8
+// waves per SIMD: it then moved some 200 of them to and from vector
+// registers in every refill.
+template <class Work>
+__device__ __forceinline__ const TravArgs<Work> &trav_args() {
+    auto p = (const __attribute__((address_space(4))) TravArgs<Work> *)
+        __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const TravArgs<Work> *)p;
+}
+
 template <int K, class Work, bool COUNT>
 __global__ void __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(COUNT ? 1 : Work::kMinWavesPerSimd, 8)))
-rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
-           uint32_t *xnext, uint4 *__restrict__ spill,
-           uint32_t spill_slots, uint32_t refill, uint32_t fin_batch,
-           uint32_t leaf_batch) {
+rti_kernel(TravArgs<Work>) {
     // stack ring: entries [K][blockDim.x], then their pending lists
     extern __shared__ uint4 ring[];
     uint32_t *const ring_st = reinterpret_cast<uint32_t *>(ring + K * blockDim.x);
-    Work work = work_arg;
-    // the unit count may come from the device (the render's block queue)
-    n = work.prepare(n);
-    // one contiguous range per XCD, or groups of xcd_group() units dealt
-    // to the XCDs in turn when the order of the units matters
-    const uint32_t xg = work.xcd_group();
-    uint32_t xch = xg ? xg : (n + kXcds - 1) / kXcds;
-    if (xch == 0) xch = 1;
     const uint32_t tid = threadIdx.x;
     const uint32_t bdim = blockDim.x;
-    const uint32_t gtid = blockIdx.x * bdim + tid;
-    const uint32_t gthreads = gridDim.x * bdim;
     const uint32_t lane = lane_id();
-    // spill buffer: entries [spill_slots][gthreads], then their lists
-    uint32_t *const spill_st =
-        reinterpret_cast<uint32_t *>(spill + (size_t)spill_slots * gthreads);
+    const uint32_t wg_waves = bdim >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t n, qf = 0, xsh, width, refill, fin_batch, leaf_batch;
+    const NodeRec *t_nodes;
+    {
+        const TravArgs<Work> &A = trav_args<Work>();
+        // the unit count may come from the device (the render's block queue)
+        n = __builtin_amdgcn_readfirstlane(A.work.prepare(A.n, qf));
+        qf = __builtin_amdgcn_readfirstlane(qf);
+        xsh = A.work.xcd_shift();
+        width = A.width;
+        refill = min(A.refill, width);
+        fin_batch = A.fin_batch;
+        leaf_batch = A.leaf_batch;
+        t_nodes = A.t.nodes;
+    }
+    // only the first `width` lanes of a wave take units (launch_shape)
+    const uint64_t lanes_used = width >= 64u ? ~0ull : (1ull << width) - 1ull;
 
     // XCD-aware hand-out: the units are cut into chunks of xch units and
-    // chunk j goes to range j % kXcds, each range with a counter of its own
-    // (own 256-byte line).  A wave draws from the range of the XCD it runs
-    // on (workgroups go round-robin over the XCDs), so neighbouring units
-    // share that XCD's L2 and no counter takes the atomics of the whole
-    // chip, and moves on to the next range when its own is used up.  With
-    // xch = n / kXcds each range is one contiguous eighth; a work type whose
-    // units are ordered longest-first deals small chunks instead, so every
-    // range follows that order.
-    uint32_t xr = blockIdx.x % kXcds, xtries = 0;
+    // chunk j goes to range j % kXcds.  A wave draws from the range of the
+    // XCD it runs on (workgroups go round-robin over the XCDs), so
+    // neighbouring units share that XCD's L2.  With xch = n / kXcds each
+    // range is one contiguous eighth; a work type whose units are ordered
+    // longest-first deals chunks of 1 << xsh instead, so every range follows
+    // that order.
+    //
+    // A wave holds a pool [pool, pool_end) of units of range xr, from which
+    // its idle lanes are refilled.  The first pools are equal shares of the
+    // range, by the wave's place in the grid; the others come from a counter
+    // per range (own 256-byte line).  A wave whose range is used up reads
+    // all counters at once and goes on with the next range that has units
+    // left; `dead` has the ranges it knows to be used up (for good: the
+    // counters only grow).  With one atomic per refill, every wave trying
+    // the 8 counters in turn at its end, and a fence there that wrote back
+    // the L2 caches, a launch without any units took 175 us; now 5.  Pools of
+    // kPool refills keep the rays of a wave neighbours: 8 M rays over 16
+    // scenes 1050 -> 820 us a launch, 16 M incoherent rays 2.19 -> 2.13 ms
+    // (8 refills: 890 us and 2.16 ms); BEST refills start 64 neighbours as
+    // it is, and larger pools only make its end longer.
+    const uint32_t xch = xsh ? 1u << xsh : max(1u, (n + kXcds - 1) / kXcds);
+    // With few refills per wave (kFew) half of the workgroups leave: the
+    // others run faster, and the last refills, which end the launch, with
+    // them (BEST work, under 8 refills: one 4K frame 466 -> 388 us, a 1080p
+    // frame close to the scene 624 -> 576; at 18 refills the full grid is
+    // faster, 1205 against 1337 us).
+    uint32_t grid = gridDim.x;
+    if (width == 64u && n / 64u / wg_waves < grid * Work::kFew)
+        grid = (grid + 1u) / 2u;
+    if (blockIdx.x >= grid) return;
+    auto waves_of = [&](uint32_t x) {
+        return ((grid + kXcds - 1u - x) / kXcds) * wg_waves;
+    };
+    auto len_of = [&](uint32_t x) {
+        const uint32_t nch = xsh ? (n + xch - 1u) >> xsh : min(n, kXcds);
+        return x < nch ? ((nch - x + kXcds - 1u) / kXcds) * xch : 0u;
+    };
+    // The first pools: an equal share of the range when that is a refill at
+    // most; else a refill, or kPool refills when that leaves three quarters
+    // of the range for later.
+    auto full = [&](uint32_t x) { return len_of(x) <= waves_of(x) * width; };
+    auto first_of = [&](uint32_t x) {
+        return len_of(x) >= waves_of(x) * (Work::kPool * 256u)
+                   ? Work::kPool * 64u : width;
+    };
+    auto shares_of = [&](uint32_t x) {
+        return full(x) ? len_of(x) : waves_of(x) * first_of(x);
+    };
+    uint32_t xr = blockIdx.x % kXcds, dead = 0, pool, pool_end;
+    for (uint32_t x = 0; x < kXcds; ++x)
+        dead |= full(x) ? 1u << x : 0u;
+    constexpr uint32_t kAllDead = (1u << kXcds) - 1u;
+    const bool counted = dead != kAllDead;
+    {
+        const uint32_t w = waves_of(xr);
+        const uint32_t share = full(xr) ? (len_of(xr) + w - 1u) / w : first_of(xr);
+        pool = min((blockIdx.x / kXcds * wg_waves + wave) * share, len_of(xr));
+        pool_end = min(pool + share, len_of(xr));
+    }
     bool active = false;
     bool exhausted = false;
     uint32_t cur = 0;
@@ -1234,31 +1364,52 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
     unsigned long long nv = 0, nt = 0, nr = 0, nl = 0, ns = 0;
 
     for (;;) {
-        uint64_t idle = __ballot(!active);
+        const uint64_t idle = __ballot(!active) & lanes_used;
         if (!exhausted && idle != 0 &&
-            (__popcll(idle) >= refill || idle == ~0ull)) {
-            uint32_t cnt = (uint32_t)__popcll(idle);
-            uint32_t leader = (uint32_t)(__ffsll((long long)idle) - 1);
-            // range x owns chunks x, x + kXcds, ... of xch units
-            const uint32_t x = xr;
-            const uint32_t nch = (n + xch - 1) / xch;
-            const uint32_t r_len =
-                x < nch ? ((nch - x + kXcds - 1) / kXcds) * xch : 0u;
-            uint32_t base = 0;
-            if (lane == leader) base = atomicAdd(&xnext[x * kXcdStride], cnt);
-            base = __shfl(base, (int)leader);
-            base = __builtin_amdgcn_readfirstlane(base);
-            if (base + cnt >= r_len) {  // range x is used up: go on to the next
-                xr = (x + 1) % kXcds;
-                if (++xtries == kXcds) exhausted = true;
+            ((uint32_t)__popcll(idle) >= refill || idle == lanes_used)) {
+            const TravArgs<Work> &A = trav_args<Work>();
+            while (pool == pool_end) {
+                if ((dead >> xr) & 1u) {
+                    if (dead != kAllDead) {
+                        const uint32_t k = lane & (kXcds - 1u);
+                        const uint32_t given =
+                            shares_of(k) +
+                            __hip_atomic_load(&global(A.xnext)[k * kXcdStride],
+                                              __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+                        dead |= (uint32_t)__ballot(given >= len_of(k)) & kAllDead;
+                    }
+                    if (dead == kAllDead) break;
+                    const uint32_t live = ~dead & kAllDead;
+                    xr = (xr + (uint32_t)__ffs((int)((live | (live << kXcds)) >> xr)) -
+                          1u) % kXcds;
+                    pool_end = shares_of(xr);  // (an estimate, for `take`)
+                }
+                // as much as leaves every wave of the range two more turns,
+                // between a refill and four
+                const uint32_t len = len_of(xr);
+                const uint32_t turn = waves_of(xr) ? waves_of(xr) * 128u : 128u;
+                const uint32_t take =
+                    width < 64u ? width
+                                : 64u * max(1u, min(Work::kPool, (len - min(len, pool_end)) / turn));
+                uint32_t base = 0;
+                if (lane == 0) base = atomicAdd(&global(A.xnext)[xr * kXcdStride], take);
+                base = __builtin_amdgcn_readfirstlane(base) + shares_of(xr);
+                pool = min(base, len);
+                pool_end = min(base + take, len);
+                if (pool == pool_end) dead |= 1u << xr;
             }
-            if (!active) {
-                const uint32_t my = base + lanes_below(idle);
-                const uint32_t u = ((my / xch) * kXcds + x) * xch + my % xch;
-                if (my < r_len && u < n) {
+            exhausted = pool == pool_end;
+            const uint32_t cnt = min((uint32_t)__popcll(idle), pool_end - pool);
+            if (!active & (lane < width)) {
+                const uint32_t rank = lanes_below(idle), my = pool + rank;
+                const uint32_t u =
+                    xsh ? ((((my >> xsh) * kXcds + xr) << xsh) | (my & (xch - 1u)))
+                        : xr * xch + my;
+                if ((rank < cnt) & (u < n)) {
                     f3 d;
-                    work.begin(u, st, cur, org, d);
-                    const Tree &T = work.tree(st, t);
+                    A.work.begin(u, qf, st, cur, org, d);
+                    const Tree &T = A.work.tree(st, A.t);
                     dir = make_dir(org, d, T.odd);
                     sp = lo = 0;
                     ph = PH_TRAV;
@@ -1274,6 +1425,7 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                     }
                 }
             }
+            pool += cnt;
         }
         if (__ballot(active) == 0) {
             if (exhausted) break;
@@ -1281,13 +1433,13 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         }
         if (!active) continue;
 
-        const Tree &T = work.tree(st, t);
+        const NodeRec *const nodes = Work::nodes(st, t_nodes);
         bool popme = false;
 
         // phase 1: one node of every traversing lane (search.c:8-29, 84-148)
         if (ph == PH_TRAV) {
             f3 e = org;
-            const Node nd = load_node(T.nodes, cur);
+            const Node nd = load_node(nodes, cur);
             if (COUNT) nv++;
             const bool in = hit_box_dir(nd.bmin, nd.bmax, org, dir, e);
             if (!in) {
@@ -1316,13 +1468,14 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                     if (sp - lo == K) {
                         // ring full: its oldest entry goes to the spill
                         // buffer (or is dropped past the bound: reported)
-                        if ((uint32_t)lo >= spill_slots) {
-                            *(volatile uint32_t *)ovf = 1u;
+                        const TravArgs<Work> &A = trav_args<Work>();
+                        if ((uint32_t)lo >= A.spill_slots) {
+                            *(volatile uint32_t *)global(A.ovf) = 1u;
                         } else {
-                            const size_t si = (size_t)lo * gthreads + gtid;
+                            const SpillSlot sl(A, wg_waves, wave, lane, lo);
                             const uint32_t ri = (lo & (K - 1)) * bdim + tid;
-                            spill[si] = ring[ri];
-                            spill_st[si] = ring_st[ri];
+                            sl.entry[0] = ring[ri];
+                            sl.list[0] = ring_st[ri];
                             if (COUNT) ns++;
                         }
                         lo++;
@@ -1348,7 +1501,9 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         // phase 2: leaves (search.c:31-81), once enough lanes wait at one
         // or no lane is traversing
         if (ph == PH_LEAF && ((uint32_t)__popcll(lm) >= leaf_batch || tm == 0)) {
-            const Node nd = load_node(T.nodes, cur);
+            const TravArgs<Work> &A = trav_args<Work>();
+            const Tree &T = A.work.tree(st, A.t);
+            const Node nd = load_node(nodes, cur);
             uint32_t vid = kEnd;
             f3 bres = org;
             const bool hit = leaf_search<COUNT>(T, nd, org, dir, vid, bres, nt);
@@ -1374,11 +1529,12 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                 // the ring is empty: the top entry comes back from the
                 // spill buffer (unless it was dropped past the bound)
                 lo--;
-                if ((uint32_t)lo < spill_slots) {
-                    const size_t si = (size_t)lo * gthreads + gtid;
+                const TravArgs<Work> &A = trav_args<Work>();
+                if ((uint32_t)lo < A.spill_slots) {
+                    const SpillSlot sl(A, wg_waves, wave, lane, lo);
                     const uint32_t ri = (lo & (K - 1)) * bdim + tid;
-                    ring[ri] = spill[si];
-                    ring_st[ri] = spill_st[si];
+                    ring[ri] = sl.entry[0];
+                    ring_st[ri] = sl.list[0];
                 } else {
                     have = false;
                 }
@@ -1393,7 +1549,7 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
                 const f3 e = f3{__uint_as_float(v.y), __uint_as_float(v.z),
                                 __uint_as_float(v.w)};
                 const uint32_t *rec =
-                    reinterpret_cast<const uint32_t *>(T.nodes + v.x);
+                    global(reinterpret_cast<const uint32_t *>(nodes + v.x));
                 const uint32_t ref = rec[offsetof(NodeRec, ref) / 4];
                 const uint32_t mask = (rec[offsetof(NodeRec, info) / 4] >> 8) & 0xffu;
                 const float cp =
@@ -1422,10 +1578,12 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         const uint64_t dm = __ballot(ph == PH_DONE);
         const uint64_t am = __ballot(true);
         if (ph == PH_DONE && ((uint32_t)__popcll(dm) >= fin_batch || dm == am)) {
+            const TravArgs<Work> &A = trav_args<Work>();
+            const Tree &T = A.work.tree(st, A.t);
             ph = T.empty ? PH_DONE : PH_TRAV;  // (an empty tree: all miss)
             sp = lo = 0;
             f3 d = dir.d;
-            if (work.finish(st, p_hit, p_vid, cur, org, cur, org, d)) {
+            if (A.work.finish(st, p_hit, p_vid, cur, org, cur, org, d)) {
                 dir = make_dir(org, d, T.odd);
                 if (COUNT) {
                     if (cur == 0) nr++;
@@ -1437,23 +1595,31 @@ rti_kernel(Tree t, Work work_arg, uint32_t n, Ctrl *ctrl, uint32_t *ovf,
         }
     }
 
+    const TravArgs<Work> &A = trav_args<Work>();
+    Ctrl *const ctrl = global(A.ctrl);
+    uint32_t *const xnext = global(A.xnext);
     if (COUNT) {
         atomicAdd(&ctrl->visits, nv);
         atomicAdd(&ctrl->tests, nt);
         atomicAdd(&ctrl->rays, nr);
         atomicAdd(&ctrl->leaf_trav, nl);
         atomicAdd(&ctrl->spills, ns);
-        work.flush(st, ctrl);
+        A.work.flush(st, ctrl);
     }
-    // self-reset of the unit counter by the last wave to leave
-    __threadfence();
+    // The last wave to leave clears the counters and, unless a later pass
+    // needs them, the queue counts; waves count themselves out per range
+    // first, so that no one address takes all of them.  Nothing has to be
+    // flushed for it: a wave's counter additions have returned by now.
+    if (!counted && A.work.keeps_queue()) return;
     if (lane == 0) {
-        uint32_t total = gridDim.x * (bdim >> 6);
-        uint32_t done = atomicAdd(&ctrl->left, 1u);
-        if (done == total - 1) {
-            for (uint32_t x = 0; x < kXcds; x++)
-                atomicExch(&xnext[x * kXcdStride], 0u);
-            if (!work.keeps_queue()) atomicExch(&ctrl->qpair, 0ull);
+        const uint32_t x = blockIdx.x % kXcds;
+        if (atomicAdd(&xnext[x * kXcdStride + 1], 1u) == waves_of(x) - 1u &&
+            atomicAdd(&ctrl->left, 1u) == min(grid, kXcds) - 1u) {
+            for (uint32_t k = 0; k < kXcds; k++) {
+                atomicExch(&xnext[k * kXcdStride], 0u);
+                atomicExch(&xnext[k * kXcdStride + 1], 0u);
+            }
+            if (!A.work.keeps_queue()) atomicExch(&ctrl->qpair, 0ull);
             atomicExch(&ctrl->left, 0u);
         }
     }
@@ -2082,7 +2248,6 @@ emit_kernel(RenderItem it, SpecOut spec, const uint32_t *__restrict__ queue,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        __threadfence();
         if (atomicAdd(&ctrl->rdone, 1u) == gridDim.x - 1u) {
             atomicExch(&ctrl->qpair, 0ull);
             atomicExch(&ctrl->rpair, 0ull);
@@ -2184,7 +2349,6 @@ emit_changed_kernel(RenderItem it, SpecOut spec,
     }
     __syncthreads();
     if (tid == 0) {
-        __threadfence();
         if (atomicAdd(&ctrl->rdone, 1u) == gridDim.x - 1u) {
             atomicExch(&ctrl->qpair, 0ull);
             atomicExch(&ctrl->rpair, 0ull);
@@ -2379,12 +2543,15 @@ namespace {
 std::mutex g_mu;
 // stack_lds, block, waves_per_cu, refill, chunk, render_cull, leaf_batch,
 // finish_batch, split_best per kind of launch (fastest measured on the
-// 256^3 benchmark scene; every field is validated by voxg_set_*)
+// 256^3 benchmark scene; every field is validated by voxg_set_*).  32 waves
+// are what a CU holds with 4 ring entries: 16 M incoherent rays take 2.12
+// ms a call with them, 2.31 with 24 and 2.71 with 16; 64 1080p BEST frames
+// 3.06, 3.29 and 3.84 ms (few refills per wave: see kFew)
 voxg_launch_config g_cfg[VOXG_LAUNCH_KINDS] = {
-    {4, 256, 32, 8, 1, 1, 24, 20, 0},   // VOXG_LAUNCH_RAYS
+    {4, 256, 32, 8, 1, 1, 24, 16, 0},   // VOXG_LAUNCH_RAYS
     {4, 256, 24, 8, 4, 1, 16, 16, 0},   // VOXG_LAUNCH_RENDER
-    {4, 256, 28, 48, 4, 1, 32, 64, 4},  // VOXG_LAUNCH_RENDER_BEST
-    {4, 256, 32, 8, 1, 1, 24, 32, 0},   // VOXG_LAUNCH_BATCH
+    {4, 256, 32, 48, 4, 1, 24, 64, 4},  // VOXG_LAUNCH_RENDER_BEST
+    {4, 256, 32, 8, 1, 1, 24, 16, 0},   // VOXG_LAUNCH_BATCH
 };
 
 voxg_launch_config current_config(int kind) {
@@ -2619,19 +2786,33 @@ dev::Tree dev_tree(const voxg_tree *t) {
     return d;
 }
 
-// Grid of a persistent traversal launch of n units: waves_per_cu waves per
-// CU, never more lanes than units (rounded up to whole workgroups; n is only
-// an upper bound when the count comes from the device).
-int traversal_grid(const voxg_launch_config &cfg, size_t n, int devid) {
-    const int cus = cu_count(devid);
-    const int block = cfg.block;
-    const int waves = std::max(1, cfg.waves_per_cu);
-    const long long threads = (long long)cus * waves * 64;
-    int grid = (int)std::max<long long>(1, threads / block);
-    long long need_blocks = ((long long)n + block - 1) / block;
-    if (need_blocks < 1) need_blocks = 1;
-    if (grid > need_blocks) grid = (int)need_blocks;
-    return grid;
+// Shape of a persistent traversal launch of n units (an upper bound when the
+// count comes from the device): waves_per_cu waves per CU, 64 lanes each,
+// when there are units for that.  A smaller launch spreads its units over
+// kSpreadWaves waves per CU, `width` lanes each: it takes as long as its
+// slowest wave, and a wave of fewer rays ends sooner (fewer iterations, and
+// fewer kinds of step in each).
+constexpr int kSpreadWaves = 8;
+struct LaunchShape {
+    int grid;
+    uint32_t width;
+    size_t lanes;  // grid's waves times width
+};
+
+LaunchShape launch_shape(const voxg_launch_config &cfg, size_t n, int devid) {
+    const size_t cus = (size_t)cu_count(devid);
+    const size_t per_wg = (size_t)cfg.block / 64;
+    const size_t most = std::max<size_t>(1, cus * (size_t)std::max(1, cfg.waves_per_cu) / per_wg);
+    const size_t spread =
+        cus * (size_t)std::min(kSpreadWaves, std::max(1, cfg.waves_per_cu));
+    const size_t width =
+        std::min<size_t>(64, std::max<size_t>(1, (n + spread - 1) / spread));
+    const size_t waves = std::max<size_t>(1, (n + width - 1) / width);
+    LaunchShape s;
+    s.grid = (int)std::min(most, (waves + per_wg - 1) / per_wg);
+    s.width = (uint32_t)width;
+    s.lanes = (size_t)s.grid * per_wg * width;
+    return s;
 }
 
 struct NoPre {
@@ -2650,12 +2831,11 @@ int launch_k(const dev::Tree &dt, uint32_t stack_bound, Work &work, size_t n,
     int devid = 0;
     HIPCHK(hipGetDevice(&devid));
     const int block = cfg.block;
-    const int grid = traversal_grid(cfg, n, devid);
-    uint32_t gthreads = (uint32_t)grid * (uint32_t)block;
+    const LaunchShape shape = launch_shape(cfg, n, devid);
     if (const uint32_t tb = g_test_bound.load()) stack_bound = std::min(stack_bound, tb);
     uint32_t slots = stack_bound > (uint32_t)K ? stack_bound - K : 0u;
     const size_t spill_need =
-        (size_t)std::max<uint32_t>(slots, 1u) * gthreads * kEntryBytes;
+        (size_t)std::max<uint32_t>(slots, 1u) * shape.lanes * kEntryBytes;
     // the stream's workspace, or one the caller owns (sized in advance)
     Workspace *ws = own;
     int rc = 0;
@@ -2681,11 +2861,11 @@ int launch_k(const dev::Tree &dt, uint32_t stack_bound, Work &work, size_t n,
     rc = pre(ws);
     if (rc) return rc;
     if (injected_failure()) return fail(VOXG_EIO, "injected failure");
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, stream, dt, work,
-                       (uint32_t)n, ws->ctrl, ws->ovf_d, ws->xnext,
-                       ws->spill, slots,
-                       (uint32_t)cfg.refill, (uint32_t)cfg.finish_batch,
-                       (uint32_t)cfg.leaf_batch);
+    const dev::TravArgs<Work> args{
+        dt, work, (uint32_t)n, ws->ctrl, ws->ovf_d, ws->xnext, ws->spill,
+        slots, shape.width, (uint32_t)cfg.refill, (uint32_t)cfg.finish_batch,
+        (uint32_t)cfg.leaf_batch};
+    hipLaunchKernelGGL(kern, dim3(shape.grid), dim3(block), lds, stream, args);
     HIPCHK(hipGetLastError());
     // the traversal's last wave clears the queue counts unless a later
     // pass still needs them
@@ -3456,7 +3636,7 @@ static int render_speculative(const voxg_tree *t, const dev::RenderItem &one,
     if (direct) {
         dev::BestDirectWork work;
         first_pass(work);
-        work.group = 256u << work.split;
+        work.group = 8u + work.split;
         rc = render_run<dev::BestDirectWork, false>(t, work, cfg, npix,
                                                     nullptr, stream);
     } else if (skip_odd) {
@@ -3464,13 +3644,13 @@ static int render_speculative(const voxg_tree *t, const dev::RenderItem &one,
         first_pass(work);
         work.pset = 1;
         work.pdiv = make_fastdiv(9);
-        work.group = 256u * 9u;
+        work.group = 11u;
         rc = render_run<dev::BestSetWork, false>(t, work, cfg, npix, nullptr,
                                                  stream);
     } else {
         dev::BestSpecWork work;
         first_pass(work);
-        work.group = 256u << work.split;
+        work.group = 8u + work.split;
         rc = render_run<dev::BestSpecWork, false>(t, work, cfg, npix, nullptr,
                                                   stream);
     }
@@ -3515,7 +3695,7 @@ static int render_speculative(const voxg_tree *t, const dev::RenderItem &one,
         first_pass(odd);
         odd.pset = 2;
         odd.pdiv = make_fastdiv(7);
-        odd.group = 256u * 7u;
+        odd.group = 11u;
         odd.queue = redo;
         odd.qpair = &ws->ctrl->rpair;
         odd.qlen = (uint32_t)nblk;
@@ -3568,7 +3748,7 @@ static int render_launch(const voxg_tree *t, size_t n_frames,
         // units dealt to the XCDs in turns of 256 blocks' worth keep the
         // longest-first order of the block queue on every XCD, and spread
         // the refill atomics over the 8 per-XCD counters
-        work.group = 256u << work.split;
+        work.group = 8u + work.split;
         return render_run<dev::BestWork, COUNT>(t, work, cfg, npix, counts,
                                                 stream);
     }
@@ -3586,7 +3766,7 @@ static int render_launch(const voxg_tree *t, size_t n_frames,
     dev::BlockWork<false> work;
     std::memset(&work, 0, sizeof(work));
     work.one = one;
-    work.group = 256u;
+    work.group = 8u;
     return render_run<dev::BlockWork<false>, COUNT>(t, work, cfg, npix,
                                                     counts, stream);
 }
@@ -3801,12 +3981,10 @@ int voxg_batch_create(size_t n_items, const voxg_batch_item *items,
     if (rc) return rc;
     // spill buffer for the launch's lanes at this configuration (the
     // largest stack_lds ring is the configured one)
-    const uint32_t gthreads =
-        (uint32_t)traversal_grid(b->cfg, b->units, devid) *
-        (uint32_t)b->cfg.block;
     const uint32_t k = (uint32_t)b->cfg.stack_lds;
     const uint32_t slots = bound > k ? bound - k : 1u;
-    const size_t sb = (size_t)slots * gthreads * kEntryBytes;
+    const size_t sb =
+        (size_t)slots * launch_shape(b->cfg, b->units, devid).lanes * kEntryBytes;
     hipError_t e = hipMalloc(&ws->spill, sb);
     if (e == hipSuccess) {
         ws->spill_bytes = sb;
