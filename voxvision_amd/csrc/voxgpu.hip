@@ -40,6 +40,7 @@
 #include <thread>
 #include <vector>
 
+#include "ball_grid.h"
 #include "cull.h"
 #include "fastdiv.h"
 #include "lights.h"
@@ -103,24 +104,56 @@ static std::vector<float> cut_of(const HostTree &h) {
     return out;
 }
 
-// HBM of an uploaded tree: node records, dots, then the cut's boxes
+// Whether the tests of raymath.h hold for the tree: its boxes, centres and
+// voxels finite, at most 2^60 in magnitude and not inverted.
+static bool plain_tree(const HostTree &h) {
+    // (a count without branches, which the compiler vectorises)
+    size_t off = 0;
+    auto far = [](float x) { return (size_t)!(std::fabs(x) <= 0x1p60f); };
+    for (const NodeRec &n : h.nodes) {
+        for (int k = 0; k < 3; k++)
+            off += far(n.bmin[k]) + far(n.bmax[k]) +
+                   (size_t)!(n.bmin[k] <= n.bmax[k]);
+        if (node_type(n.info) == NT_INNER)
+            off += far(n.c[0]) + far(n.c[1]) + far(n.c[2]);
+    }
+    for (float x : h.dots) off += far(x);
+    return off + far(h.voxel[0]) + far(h.voxel[1]) + far(h.voxel[2]) == 0;
+}
+
+// The shape of a tree's ball grid (ball_grid.h); false: none.
+static bool grid_of(const HostTree &h, bool plain, ballgrid::Grid &g) {
+    std::memset(&g, 0, sizeof(g));
+    return plain && !h.nodes.empty() && node_type(h.nodes[0].info) == NT_INNER &&
+           ballgrid::grid_shape(h.nodes[0].bmin, h.nodes[0].bmax, h.voxel,
+                                h.nodes.size(), g);
+}
+
+// HBM of an uploaded tree: node records, dots, the cut's boxes, then the
+// ball grid
 struct TreeBytes {
-    size_t dots_off, cut_off, total;
+    size_t dots_off, cut_off, grid_off, total;
 };
 
-static TreeBytes tree_bytes(const HostTree &h, size_t cut_floats) {
+static TreeBytes tree_bytes(const HostTree &h, size_t cut_floats,
+                            size_t grid_cells) {
     const size_t nb = h.nodes.size() * sizeof(NodeRec);
     const size_t db = h.dots.size() * sizeof(float);
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     TreeBytes b;
-    b.dots_off = (nb + 255) & ~(size_t)255;
-    b.cut_off = (b.dots_off + db + 255) & ~(size_t)255;
-    b.total = cut_floats ? b.cut_off + cut_floats * sizeof(float)
-                         : b.dots_off + db;
+    b.dots_off = up(nb);
+    b.cut_off = up(b.dots_off + db);
+    b.grid_off = up(b.cut_off + cut_floats * sizeof(float));
+    b.total = grid_cells ? b.grid_off + grid_cells * sizeof(uint32_t)
+              : cut_floats ? b.cut_off + cut_floats * sizeof(float)
+                           : b.dots_off + db;
     return b;
 }
 
 static size_t device_bytes_of(const HostTree &h) {
-    return tree_bytes(h, cut_of(h).size()).total;
+    ballgrid::Grid g;
+    const size_t cells = grid_of(h, plain_tree(h), g) ? ballgrid::grid_cells(g) : 0;
+    return tree_bytes(h, cut_of(h).size(), cells).total;
 }
 
 // ---------------------------------------------------------------------------
@@ -2395,74 +2428,399 @@ __device__ __forceinline__ uint8_t ball_collides(const Tree &t, f3 c, float rr,
     return 0;
 }
 
+constexpr uint32_t kGridStack = 64;  // pending nodes of grid_kernel's search
+
+// The squared distance of box_ball, for a box that is finite and not
+// inverted: the clamped coordinate is then the middle one of three (for a
+// coordinate that is not a number too: both give the lower bound).
+__device__ __forceinline__ float box_distance(f3 bmin, f3 bmax, f3 c) {
+    float dx = raymath::clamp(c.x, bmin.x, bmax.x) - c.x;
+    float dy = raymath::clamp(c.y, bmin.y, bmax.y) - c.y;
+    float dz = raymath::clamp(c.z, bmin.z, bmax.z) - c.z;
+    dx = dx * dx;
+    dy = dy * dy;
+    dz = dz * dz;
+    return (dx + dy) + dz;
+}
+
+// Fills a tree's ball grid (ball_grid.h).  A wave takes 4x4x4 cells, so
+// that its lanes walk the same nodes.  It first finds the voxel nearest to
+// the block's centre, 8 lanes testing an inner node's children and the
+// nearest of them taken first; then each lane walks, for its own cell, the
+// nodes that are nearer than grid_low of what it has, which from there are
+// few.
+__global__ void __launch_bounds__(256)
+grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out) {
+    // pending inner nodes of a wave: children and squared distance
+    __shared__ uint4 stack[4][kGridStack];
+    const uint32_t w = threadIdx.x >> 6, b = blockIdx.x * 4u + w;
+    if (b >= blocks) return;
+    const uint32_t lane = lane_id();
+    const uint32_t by = (g.n[1] + 3u) / 4u, bz = (g.n[2] + 3u) / 4u;
+    const uint32_t ix0 = b / bz / by * 4u, iy0 = b / bz % by * 4u, iz0 = b % bz * 4u;
+    const f3 mid = f3{ballgrid::grid_centre(g, 0, ix0 + 2u),
+                      ballgrid::grid_centre(g, 1, iy0 + 2u),
+                      ballgrid::grid_centre(g, 2, iz0 + 2u)};
+    const f3 V = f3{t.vx, t.vy, t.vz};
+    // the nearest voxel of a leaf to c
+    auto leaf = [&](const Node &nd, f3 c, float &best, f3 &lo, f3 &hi) {
+        if ((nd.info & NT_TYPE_MASK) == NT_DENSE) {
+            const float v = box_distance(nd.bmin, nd.bmax, c);
+            if (v < best) {
+                best = v;
+                lo = nd.bmin;
+                hi = nd.bmax;
+            }
+            return;
+        }
+        for (uint32_t k = 0; k < (nd.info >> 8); k++) {
+            const float *p = t.dots + 3u * (nd.ref + k);
+            const f3 a = f3{p[0], p[1], p[2]};
+            const f3 e = f3{a.x + V.x, a.y + V.y, a.z + V.z};
+            const float v = box_distance(a, e, c);
+            if (v < best) {
+                best = v;
+                lo = a;
+                hi = e;
+            }
+        }
+    };
+    float mid_best = INFINITY;
+    f3 lo{0, 0, 0}, hi{0, 0, 0};
+    {
+        const Node root = load_node(t.nodes, 0);
+        uint32_t sp = 1;
+        stack[w][0] = make_uint4(root.ref, (uint32_t)__popc((root.info >> 8) & 0xffu),
+                                 0u, 0u);
+        while (sp > 0) {
+            const uint4 cur = stack[w][--sp];
+            if (!(__uint_as_float(cur.z) < mid_best)) continue;
+            float dist = INFINITY, near = INFINITY;
+            f3 l{0, 0, 0}, h{0, 0, 0};
+            Node nd;
+            bool inner = false;
+            if (lane < cur.y) {
+                nd = load_node(t.nodes, cur.x + lane);
+                inner = (nd.info & NT_TYPE_MASK) == NT_INNER;
+                dist = box_distance(nd.bmin, nd.bmax, mid);
+                if (!inner && dist < mid_best) leaf(nd, mid, near, l, h);
+            }
+            // the nearest voxel of the node's leaves, over its 8 lanes
+            float m = near;
+            for (int o = 1; o < 8; o <<= 1) m = fminf(m, __shfl_xor(m, o));
+            m = __shfl(m, 0);
+            if (m < mid_best) {
+                const unsigned long long has = __ballot(near == m);
+                const int from = __ffsll((long long)has) - 1;
+                mid_best = m;
+                lo = f3{__shfl(l.x, from), __shfl(l.y, from), __shfl(l.z, from)};
+                hi = f3{__shfl(h.x, from), __shfl(h.y, from), __shfl(h.z, from)};
+            }
+            // its inner children that may hold a nearer one, nearest on top
+            const bool push = inner && dist < mid_best;
+            const uint32_t all = (uint32_t)__ballot(push);
+            uint32_t above = 0;
+            for (uint32_t k = 0; k < 8u; ++k) {
+                const float v = __shfl(dist, (int)k);
+                above += ((all >> k) & 1u) && (v > dist || (v == dist && k < lane));
+            }
+            // (a full stack drops the rest: mid_best only starts the walks)
+            if (push && sp + above < kGridStack)
+                stack[w][sp + above] =
+                    make_uint4(nd.ref, (uint32_t)__popc((nd.info >> 8) & 0xffu),
+                               __float_as_uint(dist), 0u);
+            sp = min(sp + (uint32_t)__popc(all), kGridStack);
+        }
+    }
+    const uint32_t ix = ix0 + (lane >> 4), iy = iy0 + ((lane >> 2) & 3u),
+                   iz = iz0 + (lane & 3u);
+    const f3 c = f3{ballgrid::grid_centre(g, 0, ix), ballgrid::grid_centre(g, 1, iy),
+                    ballgrid::grid_centre(g, 2, iz)};
+    // squared: to the nearest voxel so far; and what need not be looked at
+    float best = mid_best < INFINITY ? box_distance(lo, hi, c) : INFINITY;
+    float low = ballgrid::grid_low(g, best);
+    for (uint32_t node = 0; node != kEnd;) {
+        const Node nd = load_node(t.nodes, node);
+        node = nd.escape;
+        if (!(box_distance(nd.bmin, nd.bmax, c) < low)) continue;
+        if ((nd.info & NT_TYPE_MASK) != NT_INNER) {
+            leaf(nd, c, best, lo, hi);
+            low = ballgrid::grid_low(g, best);
+        } else if (nd.ref != kEnd) {
+            // (an edited tree may hold inner nodes without children)
+            node = nd.ref;
+        }
+    }
+    if ((ix < g.n[0]) & (iy < g.n[1]) & (iz < g.n[2]))
+        out[((size_t)ix * g.n[1] + iy) * g.n[2] + iz] =
+            ballgrid::grid_pack(g, low, best);
+}
+
 struct BallItem {
     Tree t;
+    ballgrid::Grid g;
     const float *cx, *cy, *cz, *r;
     uint8_t *out;
     uint32_t begin, count;  // queries [begin, begin+count) of the launch
 };
 
-template <bool COUNT, bool MULTI>
+// Counting form: the reference's search order per query (its visits and
+// tests are the counts).
 __global__ void __launch_bounds__(256)
-ball_kernel(BallItem one, const BallItem *__restrict__ items,
-            uint32_t n_items, uint32_t n, Ctrl *ctrl) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+ball_count_kernel(BallItem it, uint32_t n, Ctrl *ctrl) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     unsigned long long nv = 0, nt = 0;
     if (i < n) {
-        const BallItem *itp = &one;
-        if constexpr (MULTI) {
-            uint32_t lo = 0, hi = n_items - 1;
-            while (lo < hi) {
-                uint32_t mid = (lo + hi + 1) >> 1;
-                if (items[mid].begin <= i) lo = mid;
-                else hi = mid - 1;
+        const float r = it.r[i];
+        ball_collides<true>(it.t, f3{it.cx[i], it.cy[i], it.cz[i]}, r * r, nv, nt);
+    }
+    atomicAdd(&ctrl->visits, nv);
+    atomicAdd(&ctrl->tests, nt);
+    if (i < n) atomicAdd(&ctrl->rays, 1ull);
+}
+
+// Ball queries of one workgroup: queries [first, first + tile) of n.
+// Q gives a query's tree, grid, centre and squared radius and takes its
+// answer.
+//
+// What bounded one walk per lane (29 node visits on average for r in
+// [0.5, 8] in the 256^3 CT scene, 94 for the slowest of 64 lanes) was the
+// chain of dependent loads and the lanes that wait for the slowest.  So a
+// query is first looked up in the tree's ball grid: one load, and 89% of
+// those queries are answered.  The others are queued in LDS and taken by
+// groups of 8 lanes: an inner node's children lie side by side, a lane tests
+// one, and those that the ball touches go on the group's stack, so a query
+// takes as many steps as it touches inner nodes (7) instead of one per node
+// it looks at.  4 M queries: 618 -> 163 us (50 of them the grid), bound by
+// the latency of the children's loads, which miss the L2 a third of the
+// time; 10^4 in the 64^3 scene: 31 -> 11 us, 2.6e5 bodies 78 -> 36.  Tiles
+// of 512: with 2048 the workgroups were all resident at once and the last
+// ones ended late (220 us).  Groups of 4 lanes, two children each, took 174.
+// A grid of 64 cells an axis instead of 128 leaves twice as many queries
+// (297 us with tiles of 2048).
+constexpr uint32_t kBallTile = 512;    // most queries of a workgroup
+constexpr uint32_t kBallStack = 48;    // pending inner nodes of a group
+constexpr uint32_t kBallNone = 0xffffu;
+
+template <class Q>
+__device__ __forceinline__ void ball_tile(const Q &q, uint32_t first,
+                                          uint32_t tile, uint32_t n) {
+    __shared__ uint16_t queue[kBallTile];
+    __shared__ uint2 stack[kBallStack][32];
+    __shared__ uint32_t queued, taken;
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    if (tid == 0) queued = taken = 0;
+    __syncthreads();
+    for (uint32_t k = tid; k < tile; k += 256u) {
+        const uint32_t i = first + k;
+        bool wait = false;
+        if (i < n && q.asked(i)) {
+            f3 c;
+            float rr;
+            const Tree &t = q.tree(i);
+            const ballgrid::Grid &g = q.grid(i);
+            q.get(i, c, rr);
+            ballgrid::Verdict v = ballgrid::kUndecided;
+            size_t cell;
+            if (t.empty) v = ballgrid::kMiss;
+            else if (g.cells && ballgrid::grid_cell(g, c.x, c.y, c.z, cell))
+                v = ballgrid::grid_verdict(global(g.cells)[cell], rr);
+            else {
+                const Node nd = load_node(t.nodes, 0);
+                if (!box_ball(nd.bmin, nd.bmax, c, rr)) v = ballgrid::kMiss;
+                else if (t.odd || (nd.info & NT_TYPE_MASK) != NT_INNER) {
+                    unsigned long long a = 0, b = 0;
+                    v = (ballgrid::Verdict)ball_collides<false>(t, c, rr, a, b);
+                }
             }
-            itp = &items[lo];
+            wait = v == ballgrid::kUndecided;
+            if (!wait) q.put(i, v == ballgrid::kHit);
         }
-        const BallItem &it = *itp;
-        uint32_t k0 = i - it.begin;
-        f3 c = f3{it.cx[k0], it.cy[k0], it.cz[k0]};
-        float r = it.r[k0];
-        uint8_t res = ball_collides<COUNT>(it.t, c, r * r, nv, nt);
-        if (it.out) it.out[k0] = res;
+        const unsigned long long m = __ballot(wait);
+        if (m) {
+            const uint32_t head = (uint32_t)(__ffsll((long long)m) - 1);
+            uint32_t base = 0;
+            if (lane == head) base = atomicAdd(&queued, (uint32_t)__popcll(m));
+            base = __shfl(base, (int)head);
+            if (wait) queue[base + lanes_below(m)] = (uint16_t)k;
+        }
     }
-    if (COUNT) {
-        atomicAdd(&ctrl->visits, nv);
-        atomicAdd(&ctrl->tests, nt);
-        if (i < n) atomicAdd(&ctrl->rays, 1ull);
+    __syncthreads();
+    const uint32_t total = queued;
+    const uint32_t j = lane & 7u, shift = lane & ~7u;
+    uint2 *const st = &stack[0][tid >> 3];  // entry s at st[32 * s]
+    uint32_t k = kBallNone, sp = 0;
+    f3 c{0, 0, 0};
+    float rr = 0.0f;
+    uint2 cur = make_uint2(0, 0);  // children: first record, how many
+    const NodeRec *nodes = nullptr;
+    bool more = true;
+    for (;;) {
+        if (k == kBallNone && more) {
+            uint32_t e = 0;
+            if (j == 0) e = atomicAdd(&taken, 1u);
+            e = __shfl(e, (int)shift);
+            more = e < total;
+            if (more) {
+                k = queue[e];
+                q.get(first + k, c, rr);
+                nodes = q.tree(first + k).nodes;
+                const uint2 root =
+                    *global(reinterpret_cast<const uint2 *>(&nodes->ref));
+                cur = make_uint2(root.x, (uint32_t)__popc((root.y >> 8) & 0xffu));
+                sp = 0;
+            }
+        }
+        if (__ballot(k != kBallNone) == 0) break;
+        bool found = false, deeper = false;
+        uint2 next = make_uint2(0, 0);
+        if ((k != kBallNone) & (j < cur.y)) {
+            const float4 *p =
+                global(reinterpret_cast<const float4 *>(nodes + cur.x + j));
+            const float4 a = p[0], b = p[1];
+            if (box_distance(f3{a.x, a.y, a.z}, f3{a.w, b.x, b.y}, c) < rr) {
+                const uint32_t ref = __float_as_uint(b.z), info = __float_as_uint(b.w);
+                const uint32_t type = info & NT_TYPE_MASK;
+                deeper = type == NT_INNER;
+                next = make_uint2(ref, (uint32_t)__popc((info >> 8) & 0xffu));
+                found = type == NT_DENSE;
+                if (type == NT_LEAF) {
+                    const Tree &t = q.tree(first + k);
+                    const float *dot = global(t.dots) + 3u * ref;
+                    for (uint32_t x = 0; x < (info >> 8) && !found; x++) {
+                        const f3 v = f3{dot[3 * x], dot[3 * x + 1], dot[3 * x + 2]};
+                        found = box_distance(
+                                    v, f3{v.x + t.vx, v.y + t.vy, v.z + t.vz},
+                                    c) < rr;
+                    }
+                }
+            }
+        }
+        const uint32_t hit = (uint32_t)(__ballot(found) >> shift) & 0xffu;
+        const uint32_t in = (uint32_t)(__ballot(deeper) >> shift) & 0xffu;
+        if (k != kBallNone) {
+            const uint32_t add = (uint32_t)__popc(in);
+            int answer = hit ? 1 : -1;
+            if (answer < 0 && sp + add > kBallStack) {
+                // a stack deeper than this: one walk by the group's lanes
+                unsigned long long x = 0, y = 0;
+                answer = ball_collides<false>(q.tree(first + k), c, rr, x, y);
+            }
+            if (answer < 0) {
+                if (deeper)
+                    st[32u * (sp + (uint32_t)__popc(in & ((1u << j) - 1u)))] = next;
+                sp += add;
+                if (sp == 0) answer = 0;
+                else cur = st[32u * --sp];
+            }
+            if (answer >= 0) {
+                if (j == 0) q.put(first + k, answer != 0);
+                k = kBallNone;
+            }
+        }
     }
+}
+
+struct BallOne {
+    BallItem it;
+    __device__ __forceinline__ bool asked(uint32_t) const { return true; }
+    __device__ __forceinline__ const Tree &tree(uint32_t) const { return it.t; }
+    __device__ __forceinline__ const ballgrid::Grid &grid(uint32_t) const {
+        return it.g;
+    }
+    __device__ __forceinline__ void get(uint32_t i, f3 &c, float &rr) const {
+        c = f3{it.cx[i], it.cy[i], it.cz[i]};
+        const float r = it.r[i];
+        rr = r * r;
+    }
+    __device__ __forceinline__ void put(uint32_t i, bool hit) const {
+        it.out[i] = hit;
+    }
+};
+
+__global__ void __launch_bounds__(256)
+ball_kernel(BallOne q, uint32_t tile, uint32_t n) {
+    ball_tile(q, blockIdx.x * tile, tile, n);
+}
+
+// Ball batches of several trees (the serving loop): a query finds its item
+// by binary search over the items' first queries.
+struct BallMany {
+    const BallItem *items;
+    uint32_t n_items;
+    __device__ __forceinline__ const BallItem &item(uint32_t i) const {
+        uint32_t lo = 0, hi = n_items - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (global(items)[mid].begin <= i) lo = mid;
+            else hi = mid - 1;
+        }
+        return global(items)[lo];
+    }
+    __device__ __forceinline__ bool asked(uint32_t) const { return true; }
+    __device__ __forceinline__ const Tree &tree(uint32_t i) const { return item(i).t; }
+    __device__ __forceinline__ const ballgrid::Grid &grid(uint32_t i) const {
+        return item(i).g;
+    }
+    __device__ __forceinline__ void get(uint32_t i, f3 &c, float &rr) const {
+        const BallItem &it = item(i);
+        const uint32_t k = i - it.begin;
+        c = f3{global(it.cx)[k], global(it.cy)[k], global(it.cz)[k]};
+        const float r = global(it.r)[k];
+        rr = r * r;
+    }
+    __device__ __forceinline__ void put(uint32_t i, bool hit) const {
+        const BallItem &it = item(i);
+        if (it.out) global(it.out)[i - it.begin] = hit;
+    }
+};
+
+__global__ void __launch_bounds__(256)
+ball_multi_kernel(BallMany q, uint32_t tile, uint32_t n) {
+    ball_tile(q, blockIdx.x * tile, tile, n);
 }
 
 // cd.c:38-55 for n bodies: a body that moved (vox_dot_equalp,
 // voxvision.h.in:52: x, y and z all compare equal) and whose ball collides
 // with the scene goes back to its last position; otherwise its last
 // position becomes its position.
-__global__ void __launch_bounds__(256)
-collide_kernel(Tree t, uint32_t n, float *__restrict__ px,
-               float *__restrict__ py, float *__restrict__ pz,
-               float *__restrict__ lx, float *__restrict__ ly,
-               float *__restrict__ lz, const float *__restrict__ radius,
-               uint8_t *__restrict__ collided) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const f3 p = f3{px[i], py[i], pz[i]};
-    const f3 l = f3{lx[i], ly[i], lz[i]};
-    uint8_t moved_back = 0;
-    if (!(p.x == l.x && p.y == l.y && p.z == l.z)) {
-        const float r = radius[i];
-        unsigned long long nv = 0, nt = 0;
-        if (ball_collides<false>(t, p, r * r, nv, nt)) {
-            px[i] = l.x;
-            py[i] = l.y;
-            pz[i] = l.z;
-            moved_back = 1;
-        } else {
-            lx[i] = p.x;
-            ly[i] = p.y;
-            lz[i] = p.z;
-        }
+struct Bodies {
+    Tree t;
+    ballgrid::Grid g;
+    float *px, *py, *pz, *lx, *ly, *lz;
+    const float *radius;
+    uint8_t *collided;
+    __device__ __forceinline__ bool asked(uint32_t i) const {
+        const bool moved = !(px[i] == lx[i] && py[i] == ly[i] && pz[i] == lz[i]);
+        if (!moved && collided) collided[i] = 0;
+        return moved;
     }
-    if (collided) collided[i] = moved_back;
+    __device__ __forceinline__ const Tree &tree(uint32_t) const { return t; }
+    __device__ __forceinline__ const ballgrid::Grid &grid(uint32_t) const {
+        return g;
+    }
+    __device__ __forceinline__ void get(uint32_t i, f3 &c, float &rr) const {
+        c = f3{px[i], py[i], pz[i]};
+        const float r = radius[i];
+        rr = r * r;
+    }
+    __device__ __forceinline__ void put(uint32_t i, bool hit) const {
+        if (hit) {
+            px[i] = lx[i];
+            py[i] = ly[i];
+            pz[i] = lz[i];
+        } else {
+            lx[i] = px[i];
+            ly[i] = py[i];
+            lz[i] = pz[i];
+        }
+        if (collided) collided[i] = hit;
+    }
+};
+
+__global__ void __launch_bounds__(256)
+collide_kernel(Bodies q, uint32_t tile, uint32_t n) {
+    ball_tile(q, blockIdx.x * tile, tile, n);
 }
 
 // Scratch of voxg_ray_batch_noalloc: the control record, the per-XCD unit
@@ -2501,6 +2859,7 @@ struct voxg_tree {
     float *d_cut = nullptr;
     uint32_t ncut = 0;
     bool odd = false;  // not plain (raymath.h)
+    ballgrid::Grid grid{};
     void *d_mem = nullptr;
     size_t bytes = 0;
     int device = 0;
@@ -2939,7 +3298,9 @@ int upload(voxg_tree *t) {
     } catch (const std::bad_alloc &) {
         return fail(VOXG_ENOMEM, "host allocation failed");
     }
-    const TreeBytes tb = tree_bytes(h, cut.size());
+    ballgrid::Grid g;
+    const size_t cells = grid_of(h, !t->odd, g) ? ballgrid::grid_cells(g) : 0;
+    const TreeBytes tb = tree_bytes(h, cut.size(), cells);
     t->bytes = tb.total;
     HIPCHK(hipGetDevice(&t->device));
     if (t->bytes == 0) return 0;
@@ -2954,24 +3315,18 @@ int upload(voxg_tree *t) {
         HIPCHK(hipMemcpy(t->d_cut, cut.data(), cut.size() * sizeof(float),
                          hipMemcpyHostToDevice));
     }
-    return 0;
-}
-
-// Whether the tests of raymath.h hold for the tree: its boxes, centres and
-// voxels finite, at most 2^60 in magnitude and not inverted.
-bool plain_tree(const HostTree &h) {
-    // (a count without branches, which the compiler vectorises)
-    size_t off = 0;
-    auto far = [](float x) { return (size_t)!(std::fabs(x) <= 0x1p60f); };
-    for (const NodeRec &n : h.nodes) {
-        for (int k = 0; k < 3; k++)
-            off += far(n.bmin[k]) + far(n.bmax[k]) +
-                   (size_t)!(n.bmin[k] <= n.bmax[k]);
-        if (node_type(n.info) == NT_INNER)
-            off += far(n.c[0]) + far(n.c[1]) + far(n.c[2]);
+    if (cells) {
+        uint32_t *d = (uint32_t *)((char *)t->d_mem + tb.grid_off);
+        const uint32_t blocks = (g.n[0] + 3) / 4 * ((g.n[1] + 3) / 4) *
+                                ((g.n[2] + 3) / 4);
+        hipLaunchKernelGGL(dev::grid_kernel, dim3((blocks + 3) / 4), dim3(256), 0,
+                           nullptr, dev_tree(t), g, blocks, d);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(nullptr));
+        g.cells = d;
+        t->grid = g;
     }
-    for (float x : h.dots) off += far(x);
-    return off + far(h.voxel[0]) + far(h.voxel[1]) + far(h.voxel[2]) == 0;
+    return 0;
 }
 
 int finish_tree(voxg_tree *t, voxg_tree **out) {
@@ -3103,7 +3458,7 @@ int voxg_tree_release(voxg_tree *t) {
     return 0;
 }
 
-static void fill_info(const HostTree &h, voxg_tree_info *o) {
+static void fill_info(const HostTree &h, size_t bytes, voxg_tree_info *o) {
     std::memset(o, 0, sizeof(*o));
     o->nodes = h.nodes.size();
     o->inner = h.inner;
@@ -3114,7 +3469,7 @@ static void fill_info(const HostTree &h, voxg_tree_info *o) {
     o->voxel_ids = h.voxel_ids;
     o->depth = h.depth;
     o->stack_entries = stack_bound_of(h);
-    o->device_bytes = h.nodes.empty() ? 0 : device_bytes_of(h);
+    o->device_bytes = h.nodes.empty() ? 0 : bytes;
     if (!h.nodes.empty()) {
         for (int l = 0; l < 3; l++) {
             o->bbox_min[l] = h.nodes[0].bmin[l];
@@ -3126,7 +3481,7 @@ static void fill_info(const HostTree &h, voxg_tree_info *o) {
 
 int voxg_tree_get_info(const voxg_tree *t, voxg_tree_info *o) {
     if (!t || !o) return fail(VOXG_EINVAL, "NULL argument");
-    fill_info(t->host, o);
+    fill_info(t->host, t->bytes, o);
     return 0;
 }
 
@@ -3148,7 +3503,7 @@ int voxg_tree_plan(const float *xyz, size_t n, size_t stride,
         return fail(VOXG_ENOMEM, "host allocation failed");
     }
     if (rc) return fail(rc, err);
-    if (info) fill_info(h, info);
+    if (info) fill_info(h, device_bytes_of(h), info);
     if (hash) *hash = tree_hash(h);
     return 0;
 }
@@ -3194,7 +3549,7 @@ int voxg_tree_plan_reference(const struct vox_node *root, const float voxel[3],
         return fail(VOXG_ENOMEM, "host allocation failed");
     }
     if (rc) return fail(rc, err);
-    if (info) fill_info(h, info);
+    if (info) fill_info(h, device_bytes_of(h), info);
     if (hash) *hash = tree_hash(h);
     return 0;
 }
@@ -3400,6 +3755,15 @@ int voxg_ray_batch_noalloc(const voxg_tree *t, size_t n, const float *ox,
     return rc;
 }
 
+// Queries of a workgroup: 8 workgroups per CU (what a CU holds), between a
+// wave's worth and kBallTile.
+static uint32_t ball_tile_of(size_t n) {
+    int devid = 0;
+    if (hipGetDevice(&devid) != hipSuccess) devid = 0;
+    const size_t t = (n / ((size_t)cu_count(devid) * 8) + 63) & ~(size_t)63;
+    return (uint32_t)std::min<size_t>(dev::kBallTile, std::max<size_t>(64, t));
+}
+
 static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
                        const float *cy, const float *cz, const float *r,
                        uint8_t *out, voxg_counts *counts, hipStream_t stream) {
@@ -3413,11 +3777,10 @@ static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
     Workspace *ws = nullptr;
     rc = get_ws(stream, 16, &ws);
     if (rc) return rc;
-    int block = 256;
-    int grid = (int)((n + block - 1) / block);
     dev::BallItem one;
     std::memset(&one, 0, sizeof(one));
     one.t = dev_tree(t);
+    one.g = t->grid;
     one.cx = cx;
     one.cy = cy;
     one.cz = cz;
@@ -3428,9 +3791,8 @@ static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
     if (counts) {
         HIPCHK(hipMemsetAsync(&ws->ctrl->visits, 0,
                               dev::kCounterBytes, stream));
-        hipLaunchKernelGGL((dev::ball_kernel<true, false>), dim3(grid),
-                           dim3(block), 0, stream, one, nullptr, 0u,
-                           (uint32_t)n, ws->ctrl);
+        hipLaunchKernelGGL(dev::ball_count_kernel, dim3((unsigned)((n + 255) / 256)),
+                           dim3(256), 0, stream, one, (uint32_t)n, ws->ctrl);
         HIPCHK(hipGetLastError());
         dev::Ctrl h;
         HIPCHK(hipMemcpyAsync(&h, ws->ctrl, sizeof(h), hipMemcpyDeviceToHost,
@@ -3441,9 +3803,9 @@ static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
         counts->rays = h.rays;
         return 0;
     }
-    hipLaunchKernelGGL((dev::ball_kernel<false, false>), dim3(grid),
-                       dim3(block), 0, stream, one, nullptr, 0u, (uint32_t)n,
-                       ws->ctrl);
+    const uint32_t tile = ball_tile_of(n);
+    hipLaunchKernelGGL(dev::ball_kernel, dim3(((unsigned)n + tile - 1) / tile),
+                       dim3(256), 0, stream, dev::BallOne{one}, tile, (uint32_t)n);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -3465,11 +3827,11 @@ int voxg_cd_collide_batch(const voxg_tree *t, size_t n, float *px, float *py,
     if (n == 0) return 0;
     if (!px || !py || !pz || !lx || !ly || !lz || !radius)
         return fail(VOXG_EINVAL, "body pointer is NULL");
-    const uint32_t block = 256;
-    const uint32_t grid = (uint32_t)((n + block - 1) / block);
-    hipLaunchKernelGGL(dev::collide_kernel, dim3(grid), dim3(block), 0, stream,
-                       dev_tree(t), (uint32_t)n, px, py, pz, lx, ly, lz,
-                       radius, collided);
+    const uint32_t tile = ball_tile_of(n);
+    hipLaunchKernelGGL(dev::collide_kernel, dim3(((unsigned)n + tile - 1) / tile),
+                       dim3(256), 0, stream,
+                       dev::Bodies{dev_tree(t), t->grid, px, py, pz, lx, ly, lz,
+                                   radius, collided}, tile, (uint32_t)n);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -4136,7 +4498,7 @@ struct SrvGroup {
 // stream's previous group to reach its copy, behind whatever that stream
 // still had queued, and every stream stalled meanwhile.
 constexpr int kTableSlots = 4;
-constexpr size_t kTableBytes = 1u << 20;  // item tables of one group
+constexpr size_t kTableBytes = 2u << 20;  // item tables of one group
 
 struct SrvStream {
     hipStream_t s = nullptr;
@@ -4314,6 +4676,7 @@ int srv_launch(voxg_server *s, SrvGroup &g) {
             dev::BallItem it;
             std::memset(&it, 0, sizeof(it));
             it.t = r->t;
+            it.g = r->th->grid;
             it.cx = (const float *)base;
             it.cy = it.cx + n;
             it.cz = it.cy + n;
@@ -4377,15 +4740,11 @@ int srv_launch(voxg_server *s, SrvGroup &g) {
         if (rc) return rc;
     }
     if (balls) {
-        dev::BallItem one;
-        std::memset(&one, 0, sizeof(one));
-        Workspace *ws = nullptr;
-        int rc = get_ws(ss.s, 16, &ws);
-        if (rc) return rc;
-        hipLaunchKernelGGL((dev::ball_kernel<false, true>),
-                           dim3((balls + 255) / 256), dim3(256), 0, ss.s, one,
-                           (const dev::BallItem *)(dt + o_b),
-                           (uint32_t)bitems.size(), balls, ws->ctrl);
+        const uint32_t tile = ball_tile_of(balls);
+        hipLaunchKernelGGL(dev::ball_multi_kernel,
+                           dim3((balls + tile - 1) / tile), dim3(256), 0, ss.s,
+                           dev::BallMany{(const dev::BallItem *)(dt + o_b),
+                                         (uint32_t)bitems.size()}, tile, balls);
         HIPCHK(hipGetLastError());
     }
     // results back to the callers' buffers
