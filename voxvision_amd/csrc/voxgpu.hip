@@ -38,6 +38,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "ball_grid.h"
@@ -626,6 +627,7 @@ struct ChunkWork {
     // 8 waves per SIMD (at most 64 VGPRs; it takes 54)
     static constexpr int kMinWavesPerSimd = 8;
     static constexpr uint32_t kPool = 4, kFew = 0;
+    static constexpr int kSpread = 16;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
     // XCD hand-out: one contiguous range of the units per XCD
     __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
@@ -678,6 +680,7 @@ template <class Src, class Sink>
 struct MultiWork {
     static constexpr int kMinWavesPerSimd = 8;
     static constexpr uint32_t kPool = 4, kFew = 0;
+    static constexpr int kSpread = 16;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
     __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
         Src src;
@@ -858,6 +861,7 @@ struct BlockWork {
     // render; the multi-job form would spill at that floor
     static constexpr int kMinWavesPerSimd = MULTI ? 1 : 6;
     static constexpr uint32_t kPool = 1, kFew = 0;
+    static constexpr int kSpread = 8;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return MULTI; }
     // one render's block queue is ordered longest-first (block_cull_kernel)
     RenderItem one;             // the job when !MULTI
@@ -1132,6 +1136,7 @@ struct BestWorkT {
     // 8 waves per SIMD (at most 64 VGPRs)
     static constexpr int kMinWavesPerSimd = 8;
     static constexpr uint32_t kPool = 1, kFew = 8;
+    static constexpr int kSpread = 4;
     RenderItem one;
     SpecOut spec;            // MODE 1, 2: the root searches, for
                              // resolve_kernel, instead of the job's outputs
@@ -1344,7 +1349,7 @@ rti_kernel(TravArgs<Work>) {
     // others run faster, and the last refills, which end the launch, with
     // them (BEST work, under 8 refills: one 4K frame 466 -> 388 us, a 1080p
     // frame close to the scene 624 -> 576; at 18 refills the full grid is
-    // faster, 1205 against 1337 us).
+    // faster, 1205 against 1337 us, and three quarters of it no better).
     uint32_t grid = gridDim.x;
     if (width == 64u && n / 64u / wg_waves < grid * Work::kFew)
         grid = (grid + 1u) / 2u;
@@ -1669,20 +1674,17 @@ rti_kernel(TravArgs<Work>) {
 // block that no ray can enter, or that no ray can take near a box of the
 // cut, is finished here -- every pixel is a miss in every quality mode --
 // and the others go, in block order, to the queue the traversal kernel
-// takes its blocks from.  A workgroup covers kCullTile pixels (1024
-// blocks): it marks
-// the entering blocks in LDS, compacts them with a workgroup scan and
-// reserves its queue ranges with a single 64-bit atomic (the queue
-// counters share one address, so their atomics are serialised: one per
-// workgroup of 1024 blocks keeps them off the critical path).  In counting
+// takes its blocks from.  A workgroup covers kCullBlocks blocks (kCullTile
+// pixels): it marks the entering blocks in LDS, compacts them with a
+// workgroup scan and reserves its queue ranges with a single 64-bit atomic
+// (the queue counters share one address, so their atomics are serialised:
+// one per 1024 blocks of a large call keeps them off the critical path; a
+// small call takes fewer blocks a workgroup, see render_run).  In counting
 // mode it adds what the loop would have counted for each finished block:
 // one root search per traced pixel (ADAPTIVE with ray merging traces 8 of
 // the 16 pixels of a block whose first corner misses), one node visit per
 // search, and the block's final mode.
-constexpr uint32_t kCullBlocks = 1024;
-constexpr uint32_t kCullTile = kCullBlocks * 16;
-
-template <bool COUNT>
+template <bool COUNT, uint32_t kCullBlocks>
 __global__ void __launch_bounds__(256)
 block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
                   uint32_t *__restrict__ queue, uint32_t qlen) {
@@ -1700,6 +1702,7 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
         ndeep = 0;
     }
     __syncthreads();
+    constexpr uint32_t kCullTile = kCullBlocks * 16u, kEach = kCullBlocks / 256u;
     const uint32_t tile0 = blockIdx.x * kCullTile;
     uint32_t my_missed = 0;
     // the host launches this kernel only for a tree with a root record
@@ -1750,7 +1753,7 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
     // ray, which a deeper test would not match)
     const bool deep = !COUNT && it.t.ncut != 0;
     // one thread per block, 4 blocks per thread
-    for (uint32_t j = 0; j < kCullBlocks / 256; ++j) {
+    for (uint32_t j = 0; j < kEach; ++j) {
         const uint32_t lb = j * 256 + tid;
         const uint32_t blk = (tile0 >> 4) + lb;
         const bool valid = blk * 16u < npix;
@@ -1895,7 +1898,7 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
                             cut_box(fs, (uint32_t)(__ffsll((long long)m) - 1)), r);
                 }
                 if (!keep) {
-                    const uint32_t lb = e & 0x3ffu;
+                    const uint32_t lb = e & 0x7fffu;
                     enter[lb] = 0;
                     if (vox && !vox16) {
                         uint32_t *v = vox + (size_t)((tile0 >> 4) + lb) * 16u;
@@ -1917,14 +1920,14 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
         }
     }
     __syncthreads();
-    // ordered compaction of the 1024 block flags (thread t owns blocks
-    // 4t..4t+3): blocks whose rays all enter go to the front of the queue,
+    // ordered compaction of the block flags (thread t owns kEach blocks
+    // from kEach * t): blocks whose rays all enter go to the front of the queue,
     // the other entering blocks to the back, so the longest work is handed
     // out first and the end of the launch is made of the cheaper blocks.
     // Both counts are scanned at once, packed in the two halves of a word.
-    uint32_t cls[4], mine = 0;
-    for (uint32_t j = 0; j < 4; ++j) {
-        cls[j] = enter[4 * tid + j];
+    uint32_t cls[kEach], mine = 0;
+    for (uint32_t j = 0; j < kEach; ++j) {
+        cls[j] = enter[kEach * tid + j];
         mine += cls[j] == 2 ? 1u : (cls[j] == 1 ? 0x10000u : 0u);
     }
     uint32_t incl = mine;
@@ -1955,8 +1958,8 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
     // the counts start at 0 unless a render failed after its pre-pass:
     // entries beyond the queue are then dropped (the readers clamp the
     // counts), never written out of bounds
-    for (uint32_t j = 0; j < 4; ++j) {
-        const uint32_t id = tile0 / 16 + 4 * tid + j;
+    for (uint32_t j = 0; j < kEach; ++j) {
+        const uint32_t id = tile0 / 16 + kEach * tid + j;
         if (cls[j] == 2 && of < qlen) queue[of] = id;
         if (cls[j] == 1 && ob < qlen) queue[qlen - 1u - ob] = id;
         of += cls[j] == 2;
@@ -3148,24 +3151,30 @@ dev::Tree dev_tree(const voxg_tree *t) {
 // Shape of a persistent traversal launch of n units (an upper bound when the
 // count comes from the device): waves_per_cu waves per CU, 64 lanes each,
 // when there are units for that.  A smaller launch spreads its units over
-// kSpreadWaves waves per CU, `width` lanes each: it takes as long as its
-// slowest wave, and a wave of fewer rays ends sooner (fewer iterations, and
-// fewer kinds of step in each).
-constexpr int kSpreadWaves = 8;
+// `spread` waves per CU, `width` lanes each: it takes as long as its slowest
+// wave, and a wave of fewer rays ends sooner (fewer iterations, fewer kinds
+// of step in each), until the waves of a SIMD slow each other down.  Over 8
+// lanes the width is a multiple of the 16 pixels of a block.  Measured per
+// work type (kSpread): 20,000 rays take 70 us with 16 waves per CU, 82 with 8
+// and 93 with all lanes used; a 320x240 BEST frame from inside the 256^3
+// scene, whose neighbouring rays stay together, 72 us with 4, 86 with 8, 101
+// with 16.
 struct LaunchShape {
     int grid;
     uint32_t width;
     size_t lanes;  // grid's waves times width
 };
 
-LaunchShape launch_shape(const voxg_launch_config &cfg, size_t n, int devid) {
+LaunchShape launch_shape(const voxg_launch_config &cfg, int spread_waves,
+                         size_t n, int devid) {
     const size_t cus = (size_t)cu_count(devid);
     const size_t per_wg = (size_t)cfg.block / 64;
     const size_t most = std::max<size_t>(1, cus * (size_t)std::max(1, cfg.waves_per_cu) / per_wg);
     const size_t spread =
-        cus * (size_t)std::min(kSpreadWaves, std::max(1, cfg.waves_per_cu));
-    const size_t width =
+        cus * (size_t)std::min(spread_waves, std::max(1, cfg.waves_per_cu));
+    size_t width =
         std::min<size_t>(64, std::max<size_t>(1, (n + spread - 1) / spread));
+    if (width > 8) width = (width + 15) & ~(size_t)15;
     const size_t waves = std::max<size_t>(1, (n + width - 1) / width);
     LaunchShape s;
     s.grid = (int)std::min(most, (waves + per_wg - 1) / per_wg);
@@ -3190,7 +3199,7 @@ int launch_k(const dev::Tree &dt, uint32_t stack_bound, Work &work, size_t n,
     int devid = 0;
     HIPCHK(hipGetDevice(&devid));
     const int block = cfg.block;
-    const LaunchShape shape = launch_shape(cfg, n, devid);
+    const LaunchShape shape = launch_shape(cfg, Work::kSpread, n, devid);
     if (const uint32_t tb = g_test_bound.load()) stack_bound = std::min(stack_bound, tb);
     uint32_t slots = stack_bound > (uint32_t)K ? stack_bound - K : 0u;
     const size_t spill_need =
@@ -3927,10 +3936,23 @@ static int render_run(const voxg_tree *t, Work &work,
             HIPCHK(hipMemsetAsync(&w->ctrl->visits, 0, dev::kCounterBytes,
                                   stream));
         w->dirty = true;
-        hipLaunchKernelGGL((dev::block_cull_kernel<COUNT>),
-                           dim3((npix + dev::kCullTile - 1) / dev::kCullTile),
-                           dim3(256), 0, stream, work.one, (uint32_t)npix,
-                           w->ctrl, w->queue, (uint32_t)nblk);
+        // Blocks of a workgroup: 1024, one atomic on the queue counts for
+        // each 1024 blocks of a large call (64 1080p frames: 8100); 256 or
+        // 512 where the launch would be a few long workgroups (a 320x240
+        // frame 33 -> 21 us, a 1080p frame 34 -> 16, a 4K frame 27 -> 21).
+        auto cull = [&](auto tile) {
+            constexpr uint32_t kBlocks = decltype(tile)::value;
+            hipLaunchKernelGGL((dev::block_cull_kernel<COUNT, kBlocks>),
+                               dim3((unsigned)((nblk + kBlocks - 1) / kBlocks)),
+                               dim3(256), 0, stream, work.one, (uint32_t)npix,
+                               w->ctrl, w->queue, (uint32_t)nblk);
+        };
+        if (nblk <= 1024u * 256u)
+            cull(std::integral_constant<uint32_t, 256>());
+        else if (nblk <= 1024u * 1024u)
+            cull(std::integral_constant<uint32_t, 512>());
+        else
+            cull(std::integral_constant<uint32_t, 1024>());
         HIPCHK(hipGetLastError());
         work.queue = w->queue;
         work.qpair = &w->ctrl->qpair;
@@ -4346,7 +4368,9 @@ int voxg_batch_create(size_t n_items, const voxg_batch_item *items,
     const uint32_t k = (uint32_t)b->cfg.stack_lds;
     const uint32_t slots = bound > k ? bound - k : 1u;
     const size_t sb =
-        (size_t)slots * launch_shape(b->cfg, b->units, devid).lanes * kEntryBytes;
+        (size_t)slots *
+        launch_shape(b->cfg, dev::MultiWork<dev::SoaSrc, dev::SoaSink>::kSpread,
+                     b->units, devid).lanes * kEntryBytes;
     hipError_t e = hipMalloc(&ws->spill, sb);
     if (e == hipSuccess) {
         ws->spill_bytes = sb;
