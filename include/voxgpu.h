@@ -152,6 +152,16 @@ int voxg_ray_batch(const voxg_tree *tree, size_t n, const float *ox,
                    uint32_t *leaf_out, float *hx, float *hy, float *hz,
                    hipStream_t stream);
 
+/* voxg_ray_batch over rays stored as rows: o and d are n rows of three
+ * floats, the ids are written as 64-bit words (VOXG_MISS as 0xffffffff), and
+ * with nan_miss set the hit point of a missed ray is NaN instead of left
+ * untouched.  voxel_out, leaf_out and hx, hy, hz may be NULL; the outputs
+ * must not overlap o and d. */
+int voxg_ray_batch_rows(const voxg_tree *tree, size_t n, const float *o,
+                        const float *d, uint64_t *voxel_out,
+                        uint64_t *leaf_out, float *hx, float *hy, float *hz,
+                        int nan_miss, hipStream_t stream);
+
 /* voxg_ray_batch for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  Same arguments and results as
@@ -174,6 +184,9 @@ int voxg_ray_batch_noalloc(const voxg_tree *tree, size_t n, const float *ox,
 int voxg_ball_batch(const voxg_tree *tree, size_t n, const float *cx,
                     const float *cy, const float *cz, const float *r,
                     uint8_t *out, hipStream_t stream);
+/* voxg_ball_batch over centres stored as n rows of three floats. */
+int voxg_ball_batch_rows(const voxg_tree *tree, size_t n, const float *c,
+                         const float *r, uint8_t *out, hipStream_t stream);
 
 /* Editable host trees (vox_insert_voxel / vox_delete_voxel,
  * src/voxtrees/tree.h:96,114, tree.c:437-835).  The tree lives in host

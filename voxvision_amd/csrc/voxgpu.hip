@@ -479,6 +479,39 @@ struct SoaSink {
     }
 };
 
+// Rays as rows of three floats, ids as the 64-bit words that a caller
+// without 32-bit unsigned arrays keeps, hits of missed rays NaN on request
+// (voxg_ray_batch_rows).  The kernel reads and writes the caller's arrays:
+// two transposes, two fills and two conversions around it took 390 us of
+// 2147 for 2^24 rays into a 256^3 CT scene (1824 with this), and six
+// launches for any number (4096 rays 49 -> 30 us).
+struct RowSrc {
+    const float *o, *d;
+    __device__ __forceinline__ void get(uint32_t r, f3 &org, f3 &dir) const {
+        const auto *a = global(o) + 3ull * r;
+        const auto *b = global(d) + 3ull * r;
+        org = f3{a[0], a[1], a[2]};
+        dir = f3{b[0], b[1], b[2]};
+    }
+};
+
+struct RowSink {
+    uint64_t *voxel, *leaf;
+    float *hx, *hy, *hz;
+    uint32_t nan_miss;
+    __device__ __forceinline__ void put(uint32_t r, bool hit, uint32_t vid,
+                                        uint32_t leafi, f3 p) const {
+        if (voxel) global(voxel)[r] = hit ? vid : kEnd;
+        if (leaf) global(leaf)[r] = hit ? leafi : kEnd;
+        if (hx && (hit || nan_miss)) {
+            const float nan = __builtin_nanf("");
+            global(hx)[r] = hit ? p.x : nan;
+            global(hy)[r] = hit ? p.y : nan;
+            global(hz)[r] = hit ? p.z : nan;
+        }
+    }
+};
+
 struct CamDev {
     float px, py, pz, qw, qi, qj, qk, mul, xsub, ysub, fov;
 };
@@ -2724,15 +2757,20 @@ __device__ __forceinline__ void ball_tile(const Q &q, uint32_t first,
     }
 }
 
+// The coordinates of query i are at [i * step]: 1 for three arrays, 3 for
+// rows of three floats (with their transpose 2^22 queries of a 256^3 CT scene
+// took 220 us, 182 without it; 10,000 queries 18 and 11).
 struct BallOne {
     BallItem it;
+    uint32_t step;
     __device__ __forceinline__ bool asked(uint32_t) const { return true; }
     __device__ __forceinline__ const Tree &tree(uint32_t) const { return it.t; }
     __device__ __forceinline__ const ballgrid::Grid &grid(uint32_t) const {
         return it.g;
     }
     __device__ __forceinline__ void get(uint32_t i, f3 &c, float &rr) const {
-        c = f3{it.cx[i], it.cy[i], it.cz[i]};
+        const uint64_t k = (uint64_t)i * step;
+        c = f3{it.cx[k], it.cy[k], it.cz[k]};
         const float r = it.r[i];
         rr = r * r;
     }
@@ -3684,6 +3722,24 @@ int voxg_ray_batch(const voxg_tree *t, size_t n, const float *ox,
                                          (n + c - 1) / c, stream, nullptr);
 }
 
+int voxg_ray_batch_rows(const voxg_tree *t, size_t n, const float *o,
+                        const float *d, uint64_t *voxel_out,
+                        uint64_t *leaf_out, float *hx, float *hy, float *hz,
+                        int nan_miss, hipStream_t stream) {
+    int rc = ray_common(t, n, o, o, o, d, d, d);
+    if (rc) return rc;
+    if ((hx || hy || hz) && !(hx && hy && hz))
+        return fail(VOXG_EINVAL, "hx, hy, hz must be all set or all NULL");
+    if (n == 0) return 0;
+    uint32_t c = effective_chunk(n, VOXG_LAUNCH_RAYS);
+    dev::ChunkWork<dev::RowSrc, dev::RowSink> work{
+        dev::RowSrc{o, d},
+        dev::RowSink{voxel_out, leaf_out, hx, hy, hz, nan_miss != 0},
+        (uint32_t)n, c};
+    return launch<decltype(work), false>(VOXG_LAUNCH_RAYS, t, work,
+                                         (n + c - 1) / c, stream, nullptr);
+}
+
 int voxg_ray_batch_count(const voxg_tree *t, size_t n, const float *ox,
                          const float *oy, const float *oz, const float *dx,
                          const float *dy, const float *dz, voxg_counts *out,
@@ -3774,8 +3830,9 @@ static uint32_t ball_tile_of(size_t n) {
 }
 
 static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
-                       const float *cy, const float *cz, const float *r,
-                       uint8_t *out, voxg_counts *counts, hipStream_t stream) {
+                       const float *cy, const float *cz, uint32_t step,
+                       const float *r, uint8_t *out, voxg_counts *counts,
+                       hipStream_t stream) {
     int rc = check_tree(t);
     if (rc) return rc;
     if (n >= 0x80000000ull) return fail(VOXG_ERANGE, "n must be < 2^31");
@@ -3814,7 +3871,8 @@ static int ball_launch(const voxg_tree *t, size_t n, const float *cx,
     }
     const uint32_t tile = ball_tile_of(n);
     hipLaunchKernelGGL(dev::ball_kernel, dim3(((unsigned)n + tile - 1) / tile),
-                       dim3(256), 0, stream, dev::BallOne{one}, tile, (uint32_t)n);
+                       dim3(256), 0, stream, dev::BallOne{one, step}, tile,
+                       (uint32_t)n);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -3823,7 +3881,14 @@ int voxg_ball_batch(const voxg_tree *t, size_t n, const float *cx,
                     const float *cy, const float *cz, const float *r,
                     uint8_t *out, hipStream_t stream) {
     if (n && !out) return fail(VOXG_EINVAL, "out is NULL");
-    return ball_launch(t, n, cx, cy, cz, r, out, nullptr, stream);
+    return ball_launch(t, n, cx, cy, cz, 1, r, out, nullptr, stream);
+}
+
+int voxg_ball_batch_rows(const voxg_tree *t, size_t n, const float *c,
+                         const float *r, uint8_t *out, hipStream_t stream) {
+    if (n && !out) return fail(VOXG_EINVAL, "out is NULL");
+    return ball_launch(t, n, c, c ? c + 1 : nullptr, c ? c + 2 : nullptr, 3, r,
+                       out, nullptr, stream);
 }
 
 int voxg_cd_collide_batch(const voxg_tree *t, size_t n, float *px, float *py,
@@ -3850,7 +3915,7 @@ int voxg_ball_batch_count(const voxg_tree *t, size_t n, const float *cx,
                           voxg_counts *out, hipStream_t stream) {
     if (!out) return fail(VOXG_EINVAL, "out is NULL");
     std::memset(out, 0, sizeof(*out));
-    return ball_launch(t, n, cx, cy, cz, r, nullptr, out, stream);
+    return ball_launch(t, n, cx, cy, cz, 1, r, nullptr, out, stream);
 }
 
 static int render_common(const voxg_tree *t, size_t n_frames,

@@ -32,6 +32,16 @@ def _dev_f32(x, n=None, cols=None):
     return t
 
 
+def _rows(x, stream):
+    """x as n rows of three floats on the device.  A call on another stream
+    than the current one reads a copy: the caller may go on writing x."""
+    t = _dev_f32(x).reshape(-1, 3)
+    if stream is not None and \
+            stream.cuda_stream != torch.cuda.current_stream().cuda_stream:
+        t = t.clone()
+    return t
+
+
 class Tree:
     """A flattened tree resident in device memory (immutable)."""
 
@@ -140,32 +150,31 @@ def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
     Returns (voxel_id uint32-as-int64 tensor, hit (3, n) float32 tensor
     [, leaf node index tensor])."""
     L = _lib.load()
-    o = _dev_f32(o).reshape(-1, 3)
-    d = _dev_f32(d).reshape(-1, 3)
+    o = _rows(o, stream)
+    d = _rows(d, stream)
     n = o.shape[0]
-    oc = o.t().contiguous()
-    dc = d.t().contiguous()
-    # every traced ray overwrites its entry (an id or VOXG_MISS); -2 marks
-    # a ray that was not traced
-    vox = torch.full((n,), -2, dtype=torch.int32, device="cuda")
-    leaf = torch.empty(n, dtype=torch.int32, device="cuda") if want_leaf \
+    if d.shape[0] < n:
+        raise ValueError("a direction for every origin")
+    # the library writes every ray's id (VOXG_MISS is 0xffffffff), and a
+    # missed ray's hit only where there is no hit_init
+    vox = torch.empty(n, dtype=torch.int64, device="cuda")
+    leaf = torch.empty(n, dtype=torch.int64, device="cuda") if want_leaf \
         else None
-    if hit_init is None:
-        hit = torch.full((3, n), float("nan"), dtype=torch.float32,
-                         device="cuda")
-    else:
-        hit = hit_init
-    check(L.voxg_ray_batch(tree.handle, n, oc[0].data_ptr(),
-                           oc[1].data_ptr(), oc[2].data_ptr(),
-                           dc[0].data_ptr(), dc[1].data_ptr(),
-                           dc[2].data_ptr(), vox.data_ptr(),
-                           leaf.data_ptr() if leaf is not None else None,
-                           hit[0].data_ptr(), hit[1].data_ptr(),
-                           hit[2].data_ptr(), _stream(stream)),
-          "voxg_ray_batch")
-    vox = vox.to(torch.int64) & 0xFFFFFFFF
+    hit = hit_init
+    if hit is None:
+        hit = torch.empty((3, n), dtype=torch.float32, device="cuda")
+    else:  # hits are written while other rays are read
+        o, d = (x.clone() if x.untyped_storage().data_ptr() ==
+                hit.untyped_storage().data_ptr() else x for x in (o, d))
+    check(L.voxg_ray_batch_rows(tree.handle, n, o.data_ptr(), d.data_ptr(),
+                                vox.data_ptr(),
+                                leaf.data_ptr() if want_leaf else None,
+                                hit[0].data_ptr(), hit[1].data_ptr(),
+                                hit[2].data_ptr(), hit_init is None,
+                                _stream(stream)),
+          "voxg_ray_batch_rows")
     if want_leaf:
-        return vox, hit, leaf.to(torch.int64) & 0xFFFFFFFF
+        return vox, hit, leaf
     return vox, hit
 
 
@@ -187,13 +196,15 @@ def ray_counts(tree, o, d, stream=None):
 def tree_ball_collidep(tree, c, r, stream=None):
     """Batched vox_tree_ball_collidep: (n,3) centres, (n,) radii -> uint8."""
     L = _lib.load()
-    c = _dev_f32(c).reshape(-1, 3).t().contiguous()
-    r = _dev_f32(r).reshape(-1).contiguous()
-    n = c.shape[1]
+    c = _rows(c, stream)
+    r = _dev_f32(r).reshape(-1)
+    n = c.shape[0]
+    if r.shape[0] < n:
+        raise ValueError("a radius for every centre")
     out = torch.empty(n, dtype=torch.uint8, device="cuda")
-    check(L.voxg_ball_batch(tree.handle, n, c[0].data_ptr(), c[1].data_ptr(),
-                            c[2].data_ptr(), r.data_ptr(), out.data_ptr(),
-                            _stream(stream)), "voxg_ball_batch")
+    check(L.voxg_ball_batch_rows(tree.handle, n, c.data_ptr(), r.data_ptr(),
+                                 out.data_ptr(), _stream(stream)),
+          "voxg_ball_batch_rows")
     return out
 
 
