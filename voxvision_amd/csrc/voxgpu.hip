@@ -782,11 +782,16 @@ __device__ __forceinline__ float sqr_metric(f3 a, f3 b) {
 // box at e, hits first: a dense leaf's voxel at e, or the voxel whose entry
 // point is L1-closest to e (strictly, in stored order; an entry at e ends
 // the search).  Writes the voxel id and the hit point; false: no voxel.
-template <bool COUNT, bool PREFETCH = false>
+// With PREFETCH the corners of the first 7 voxels (a leaf's most, except an
+// overflow leaf's) come from `first(k)`.
+struct NoDots {};
+
+template <bool COUNT, bool PREFETCH = false, class First = NoDots>
 __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
                                             f3 e, const Dir &d, uint32_t &vid,
                                             f3 &bres,
-                                            unsigned long long &nt) {
+                                            unsigned long long &nt,
+                                            First first = First{}) {
     bres = e;
     if ((nd.info & NT_TYPE_MASK) == NT_DENSE) {
         vid = dense_voxel(nd, e, T);
@@ -800,21 +805,22 @@ __device__ __forceinline__ bool leaf_search(const Tree &T, const Node &nd,
     if constexpr (PREFETCH) {
         // the first 7 voxels' corners loaded together, not one round trip
         // per voxel
-        float qx[7], qy[7], qz[7];
-        const float *base = global(T.dots) + 3u * nd.ref;
+        f3 q[7];
+        const auto *base = global(T.dots) + 3u * nd.ref;
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
-            qx[k] = qy[k] = qz[k] = 0.0f;
+            q[k] = f3{0.0f, 0.0f, 0.0f};
             if ((uint32_t)k < cnt) {
-                qx[k] = base[3 * k];
-                qy[k] = base[3 * k + 1];
-                qz[k] = base[3 * k + 2];
+                if constexpr (std::is_same<First, NoDots>::value)
+                    q[k] = f3{base[3 * k], base[3 * k + 1], base[3 * k + 2]};
+                else
+                    q[k] = first(k);
             }
         }
 #pragma unroll
         for (int k = 0; k < 7; ++k) {
             if ((uint32_t)k < cnt) {
-                f3 vmin = f3{qx[k], qy[k], qz[k]};
+                f3 vmin = q[k];
                 f3 vmax = f3{vmin.x + V.x, vmin.y + V.y, vmin.z + V.z};
                 f3 far;
                 if (COUNT) nt++;
@@ -2257,6 +2263,174 @@ resolve_kernel(RenderItem it, SpecOut spec, const uint32_t *__restrict__ queue,
             } else {
                 leaf = kEnd;
             }
+        }
+    }
+}
+
+// The same for a direct render of at most kSmallBlocks blocks, with 16 lanes
+// per block, lane j the block's j-th pixel in the reference's order.  The
+// chain of a block changes its leaf only where a try fails, so that a round
+// tries the current leaf with every pixel still to come at once: the pixels
+// before the first that fails keep the leaf, and that pixel's own leaf is
+// the next one.  The leaves that the chain can reach are the root searches'
+// own: each lane puts its leaf in LDS beforehand, and no round waits for
+// memory.  The pixels that changed are written straight to the outputs, a
+// block's run at a time, in place of emit_changed_kernel.
+// A thread per block waits twice for memory in each of its 15 steps: 53 us
+// on a 320x240 frame, however few its blocks, and 5 us for the output pass
+// after it.  Windows of 320x240, 640x480 and 1280x720, ADAPTIVE, from 0.3 to
+// 1.5 scene diagonals: 102 .. 253 us become 71 .. 211, 143 .. 292 become 111
+// .. 243, and 157 .. 355 become 105 .. 328.  It tries more pixels than the
+// reference's chain does: where nearly every block of a 1920x1080 frame is
+// queued (130,000) it is 2 to 13 % slower, at 1280x720 (57,600) never.
+constexpr uint32_t kSmallBlocks = 1u << 16;
+
+__global__ void __launch_bounds__(256)
+resolve_small_kernel(RenderItem it, SpecOut spec,
+                     const uint32_t *__restrict__ queue, uint32_t qlen,
+                     Ctrl *ctrl) {
+    // a leaf's record, then the corners of its first 7 voxels
+    constexpr uint32_t kRec = 33;
+    __shared__ float stage[256 * kRec];
+    uint32_t qf, qt;
+    queue_counts(ctrl->qpair, qlen, qf, qt);
+    // workgroups that have blocks; the others read the counts at any time
+    const uint32_t parts = min(gridDim.x, (qt + 15u) / 16u);
+    if (blockIdx.x >= parts) return;
+    const Tree &T = it.t;
+    const uint32_t tid = threadIdx.x, j = tid & 15u;
+    const uint32_t shift = tid & 48u;  // the block's lanes in the wave
+    const int p = render_order((int)j);
+    auto group = [&](bool x) {
+        return (uint32_t)(__ballot(x) >> shift) & 0xffffu;
+    };
+    unsigned long long nt = 0;
+    for (uint32_t b0 = blockIdx.x * 16u; b0 < qt; b0 += gridDim.x * 16u) {
+        const uint32_t b = b0 + (tid >> 4);
+        const bool have = b < qt;
+        const uint32_t id =
+            have ? queue[b < qf ? b : qlen - 1u - (b - qf)] : 0u;
+        const uint32_t nd = have ? spec.node[id * 16u + (uint32_t)p] : kEnd;
+        const uint32_t hits = group(nd != kEnd);
+        const uint32_t f = it.bpf.div(id);
+        const uint32_t cs = id - f * it.bpf.d;
+        const uint32_t row = it.ws.div(cs);
+        const int xs = (int)(cs - row * it.ws.d) * 4, ys = (int)row * 4;
+        const CamDev &c = it.cams[f];
+        const f3 o = f3{c.px, c.py, c.pz};
+        const f3 d = screen2world(c, xs + (p & 3), ys + (p >> 2));
+        // the steps at .. end - 1 are to be tried, with the leaf of lane
+        // `from` (16: none)
+        uint32_t at = 0, end = 16, from = 16;
+        bool work = hits && (it.rnd_mode == VOXG_QUALITY_FAST ||
+                             it.rnd_mode == VOXG_QUALITY_ADAPTIVE);
+        if (it.rnd_mode == VOXG_QUALITY_ADAPTIVE) {
+            // renderer.c:240-281 (pixel 15 is the last step, too)
+            at = 1;
+            if (hits & 1u) {
+                from = 0;
+                end = 15;
+                if (hits & 0x8000u) {
+                    const uint32_t k = spec.stride + id;
+                    const f3 p0 = f3{spec.cx[id], spec.cy[id], spec.cz[id]};
+                    const f3 p15 = f3{spec.cx[k], spec.cy[k], spec.cz[k]};
+                    const f3 dir1 = screen2world(c, xs, ys);
+                    const f3 dir15 = screen2world(c, xs + 3, ys + 3);
+                    const float d1 = sqr_metric(p0, o);
+                    const float d2 =
+                        (dir1.x * dir1.x + dir1.y * dir1.y) + dir1.z * dir1.z;
+                    const float criteria = d1 / d2 * sqr_metric(dir1, dir15);
+                    const float dist = sqr_metric(p0, p15);
+                    if ((double)(dist / criteria) > 1.69) work = false;
+                }
+            }
+        }
+        if (work && nd != kEnd) {
+            const Node n = load_node(T.nodes, nd);
+            float *w = stage + tid * kRec;
+            w[0] = n.bmin.x;
+            w[1] = n.bmin.y;
+            w[2] = n.bmin.z;
+            w[3] = n.bmax.x;
+            w[4] = n.bmax.y;
+            w[5] = n.bmax.z;
+            w[6] = n.c.x;
+            w[7] = n.c.y;
+            w[8] = n.c.z;
+            w[9] = __uint_as_float(n.ref);
+            w[10] = __uint_as_float(n.info);
+            if ((n.info & NT_TYPE_MASK) != NT_DENSE) {
+                const auto *q = global(T.dots) + 3u * n.ref;
+                const uint32_t cnt = n.info >> 8;
+#pragma unroll
+                for (uint32_t k = 0; k < 7u; ++k)
+                    if (k < cnt) {
+                        w[12 + 3 * k] = q[3 * k];
+                        w[13 + 3 * k] = q[3 * k + 1];
+                        w[14 + 3 * k] = q[3 * k + 2];
+                    }
+            }
+        }
+        // (a block's lanes are in one wave)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const Dir dr = make_dir(o, d, T.odd);
+        bool changed = false;
+        uint32_t cvid = kEnd;
+        f3 cpt = o;
+        while (__ballot(work)) {
+            if (work && from == 16u) {
+                // no leaf: the next step whose root search hit has one
+                const uint32_t rest = hits & (0xffffu << at);
+                from = rest ? (uint32_t)__ffs(rest) - 1u : end;
+                at = from + 1u;
+            }
+            work = work && at < end;
+            bool ok = false;
+            if (work && j >= at && j < end) {
+                const float *w = stage + ((tid & ~15u) + from) * kRec;
+                Node n;
+                n.bmin = f3{w[0], w[1], w[2]};
+                n.bmax = f3{w[3], w[4], w[5]};
+                n.c = f3{w[6], w[7], w[8]};
+                n.ref = __float_as_uint(w[9]);
+                n.info = __float_as_uint(w[10]);
+                uint32_t vid = kEnd;
+                f3 e, pt;
+                ok = hit_box_dir(n.bmin, n.bmax, o, dr, e) &&
+                     leaf_search<false, true>(
+                         T, n, e, dr, vid, pt, nt, [&](int k) {
+                             return f3{w[12 + 3 * k], w[13 + 3 * k],
+                                       w[14 + 3 * k]};
+                         });
+                if (ok) {
+                    cvid = vid;
+                    cpt = pt;
+                }
+            }
+            const uint32_t kept = group(ok);
+            if (work) {
+                const uint32_t lost =
+                    ((1u << end) - 1u) & (0xffffu << at) & ~kept;
+                const uint32_t first =
+                    lost ? (uint32_t)__ffs(lost) - 1u : end;
+                // (a later round's tries replace what this one found for
+                // the steps from `first` on)
+                if (ok && j < first) changed = true;
+                from = (hits >> first) & 1u ? first : 16u;
+                at = first + 1u;
+                work = at < end;
+            }
+        }
+        if (changed) it.sink.put(id * 16u + (uint32_t)p, true, cvid, 0, cpt);
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    if (tid == 0) {
+        if (atomicAdd(&ctrl->rdone, 1u) == parts - 1u) {
+            atomicExch(&ctrl->qpair, 0ull);
+            atomicExch(&ctrl->rpair, 0ull);
+            atomicExch(&ctrl->rdone, 0u);
         }
     }
 }
@@ -4113,20 +4287,35 @@ static int render_speculative(const voxg_tree *t, const dev::RenderItem &one,
     // modes; for the direct ones 16 for the replay (more blocks in flight
     // hide its leaf loads: 0.45 -> 0.38 ms on the benchmark frames) and 2
     // for the output pass (fewer regions in flight at a time write fewer
-    // lines at once: 0.22 -> 0.12 ms)
+    // lines at once: 0.22 -> 0.12 ms), 8 with lights, whose sums it waits
+    // for (a lit 1920x1080 frame 549 -> 525 us)
     auto wg_grid = [&](size_t per_cu) {
         return std::max<size_t>(1, std::min<size_t>((nblk + 255) / 256,
                                                     (size_t)cu_count(devid) * per_cu));
     };
     const size_t grid = wg_grid(8);
+    const bool lit = one.sink.squares && one.sink.sh.lnodes;
     if (injected_failure()) return fail(VOXG_EIO, "injected failure");
+    if (direct && nblk <= dev::kSmallBlocks) {
+        hipLaunchKernelGGL(dev::resolve_small_kernel,
+                           dim3((unsigned)((nblk + 15) / 16)), dim3(256), 0,
+                           stream, one, spec, ws->queue, (uint32_t)nblk,
+                           ws->ctrl);
+        HIPCHK(hipGetLastError());
+        if (injected_failure()) return fail(VOXG_EIO, "injected failure");
+        ws->dirty = false;
+        return 0;
+    }
     if (direct) {
         hipLaunchKernelGGL(dev::resolve_kernel<true>, dim3((unsigned)wg_grid(16)),
                            dim3(256), 0, stream, one, spec, ws->queue,
                            (uint32_t)nblk, ws->ctrl, nullptr, 0);
         HIPCHK(hipGetLastError());
         if (injected_failure()) return fail(VOXG_EIO, "injected failure");
-        hipLaunchKernelGGL(dev::emit_changed_kernel, dim3((unsigned)wg_grid(2)),
+        hipLaunchKernelGGL(dev::emit_changed_kernel,
+                           dim3((unsigned)std::min<size_t>(
+                               nreg, (size_t)cu_count(devid) *
+                                         (lit ? 8 : 2))),
                            dim3(256), 0, stream, one, spec, ws->queue,
                            (uint32_t)nblk, ws->ctrl);
         HIPCHK(hipGetLastError());
