@@ -90,7 +90,7 @@ typedef struct {
     uint32_t depth;          /* levels, root = 1 */
     uint32_t stack_entries;  /* traversal stack bound: one entry per
                                 inner level, depth-1 (at least 1) */
-    uint64_t device_bytes;   /* flattened tree size in HBM */
+    uint64_t device_bytes;   /* flattened tree and ball grid in HBM */
     float bbox_min[3], bbox_max[3];
     float voxel[3];          /* voxel size snapshot taken at build/upload */
 } voxg_tree_info;

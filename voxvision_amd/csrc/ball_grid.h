@@ -101,7 +101,8 @@ __host__ __device__ inline float grid_centre(const Grid &g, int axis, uint32_t i
 // to look when it has one at the squared distance D2: all of it within four
 // cells, and a fifth of the rest less.  Far from the voxels the exact
 // distance decides few queries, and its search looks at most of the tree
-// (2.0 ms for the 256^3 CT scene, against 0.3 with this).
+// (the 256^3 CT scene's grid: 2.0 ms without this, 1.3 with it, 0.58 with
+// grid_kernel's start from the middle of its cells as well).
 __host__ __device__ inline float grid_low(const Grid &g, float D2) {
     const float D = sqrtf(D2);
     const float low = D > 4.0f * g.h ? D - 0.2f * (D - 4.0f * g.h) : D;
