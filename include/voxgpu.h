@@ -515,8 +515,8 @@ int voxg_read_raw_data(const char *filename, const unsigned dim[3],
  *                 the 4x4 blocks whose rays all miss the scene box; 0: every
  *                 block goes through the traversal
  *   leaf_batch    lanes of a wave that wait at a leaf before the wave
- *                 searches its voxels (1..64; fewer when no lane of the wave
- *                 can go on traversing)
+ *                 searches its voxels (1..64, of 64 lanes that traverse or
+ *                 wait; fewer in proportion when fewer do)
  *   finish_batch  lanes of a wave whose traversal ended before the wave
  *                 stores their results and starts their next rays (1..64;
  *                 fewer when no other lane is left)

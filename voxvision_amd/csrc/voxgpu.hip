@@ -1575,9 +1575,15 @@ rti_kernel(TravArgs<Work>) {
         const uint64_t tm = __ballot(ph == PH_TRAV);
         const uint64_t lm = __ballot(ph == PH_LEAF);
 
-        // phase 2: leaves (search.c:31-81), once enough lanes wait at one
-        // or no lane is traversing
-        if (ph == PH_LEAF && ((uint32_t)__popcll(lm) >= leaf_batch || tm == 0)) {
+        // phase 2: leaves (search.c:31-81), once leaf_batch of 64 lanes wait
+        // at one: of those that have work, so that the few lanes left of a
+        // group, or of a launch, don't wait for a count they cannot reach
+        // until none of them traverses (a 1080p window, whose groups end
+        // with long rays, 547 -> 487 us, 16 ADAPTIVE frames 1187 -> 1146, a
+        // 4K frame 376 -> 350; where waves stay full, as in ray batches,
+        // within 1%)
+        if (ph == PH_LEAF && 64u * (uint32_t)__popcll(lm) >=
+                                 leaf_batch * (uint32_t)__popcll(tm | lm)) {
             const TravArgs<Work> &A = trav_args<Work>();
             const Tree &T = A.work.tree(st, A.t);
             const Node nd = load_node(nodes, cur);
@@ -3120,12 +3126,15 @@ std::mutex g_mu;
 // 256^3 benchmark scene; every field is validated by voxg_set_*).  32 waves
 // are what a CU holds with 4 ring entries: 16 M incoherent rays take 2.12
 // ms a call with them, 2.31 with 24 and 2.71 with 16; 64 1080p BEST frames
-// 3.06, 3.29 and 3.84 ms (few refills per wave: see kFew)
+// 3.06, 3.29 and 3.84 ms (few refills per wave: see kFew).  leaf_batch 16,
+// 24, 28, 32 and 40: incoherent rays 1833, 1778, 1761, 1758 and 1770 us, BEST
+// 3080, 3051, 3034, 3019 and 3004, one lit 1080p window 473, 487, 485, 485
+// and 500
 voxg_launch_config g_cfg[VOXG_LAUNCH_KINDS] = {
-    {4, 256, 32, 8, 1, 1, 24, 16, 0},   // VOXG_LAUNCH_RAYS
+    {4, 256, 32, 8, 1, 1, 28, 16, 0},   // VOXG_LAUNCH_RAYS
     {4, 256, 24, 8, 4, 1, 16, 16, 0},   // VOXG_LAUNCH_RENDER
-    {4, 256, 32, 48, 4, 1, 24, 64, 4},  // VOXG_LAUNCH_RENDER_BEST
-    {4, 256, 32, 8, 1, 1, 24, 16, 0},   // VOXG_LAUNCH_BATCH
+    {4, 256, 32, 48, 4, 1, 32, 64, 4},  // VOXG_LAUNCH_RENDER_BEST
+    {4, 256, 32, 8, 1, 1, 28, 16, 0},   // VOXG_LAUNCH_BATCH
 };
 
 voxg_launch_config current_config(int kind) {
