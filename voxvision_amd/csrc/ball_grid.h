@@ -22,6 +22,11 @@
 // relative, rounded outward to the 16 bits that are kept.  Squares neither
 // underflow nor overflow for boxes within 2^60 and cells of 2^-30 and more;
 // other trees get no grid.
+//
+// The search also asks that the ball touches every box above the voxel.  In a
+// tree whose boxes hold what is below them it does then (the clamp, and with
+// it each computed distance, is monotone in the box); the grid of another
+// tree decides nothing.
 #pragma once
 #include <math.h>
 #include <stddef.h>
@@ -138,6 +143,9 @@ __host__ __device__ inline bool grid_cell(const Grid &g, float x, float y,
 }
 
 enum Verdict { kMiss = 0, kHit = 1, kUndecided = 2 };
+
+// A cell that decides nothing: L2 zero, U2 infinite.
+constexpr uint32_t kNoBounds = 0x7f800000u;
 
 __host__ __device__ inline Verdict grid_verdict(uint32_t cell, float rr) {
     if (rr < bits_float(cell << 16)) return kMiss;

@@ -162,7 +162,8 @@ static TreeBytes tree_bytes(const HostTree &h, size_t cut_floats,
     b.dots_off = up(nb);
     b.cut_off = up(b.dots_off + db);
     b.grid_off = up(b.cut_off + cut_floats * sizeof(float));
-    b.total = grid_cells ? b.grid_off + grid_cells * sizeof(uint32_t)
+    // (and a word after the cells, see nested_kernel)
+    b.total = grid_cells ? b.grid_off + (grid_cells + 1) * sizeof(uint32_t)
               : cut_floats ? b.cut_off + cut_floats * sizeof(float)
                            : b.dots_off + db;
     return b;
@@ -2676,14 +2677,49 @@ __device__ __forceinline__ float box_distance(f3 bmin, f3 bmax, f3 c) {
     return (dx + dy) + dz;
 }
 
+// Whether a tree is nested: every child's box in its parent's, every voxel's
+// in its leaf's, corner by corner as the searches compute them.  Then a ball
+// that touches a voxel touches every box above it too, which is what lets the
+// grid answer by the voxels alone.  Trees that vox_make_tree and the edits
+// make are; one uploaded with larger voxels than it was built for, or made by
+// other means, need not be.  Sets *odd (zero before) if not.
+__global__ void __launch_bounds__(256)
+nested_kernel(Tree t, uint32_t nodes, uint32_t *odd) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= nodes) return;
+    const Node nd = load_node(t.nodes, i);
+    const uint32_t type = nd.info & NT_TYPE_MASK;
+    bool in = true;
+    auto inside = [&](f3 lo, f3 hi) {
+        in = in & (lo.x >= nd.bmin.x) & (lo.y >= nd.bmin.y) &
+             (lo.z >= nd.bmin.z) & (hi.x <= nd.bmax.x) & (hi.y <= nd.bmax.y) &
+             (hi.z <= nd.bmax.z);
+    };
+    if (type == NT_INNER) {
+        const uint32_t n = (uint32_t)__popc((nd.info >> 8) & 0xffu);
+        for (uint32_t k = 0; k < n; k++) {
+            const Node c = load_node(t.nodes, nd.ref + k);
+            inside(c.bmin, c.bmax);
+        }
+    } else if (type == NT_LEAF) {
+        for (uint32_t k = 0; k < (nd.info >> 8); k++) {
+            const float *p = t.dots + 3u * (nd.ref + k);
+            const f3 a = f3{p[0], p[1], p[2]};
+            inside(a, f3{a.x + t.vx, a.y + t.vy, a.z + t.vz});
+        }
+    }
+    if (!in) *odd = 1u;
+}
+
 // Fills a tree's ball grid (ball_grid.h).  A wave takes 4x4x4 cells, so
 // that its lanes walk the same nodes.  It first finds the voxel nearest to
 // the block's centre, 8 lanes testing an inner node's children and the
 // nearest of them taken first; then each lane walks, for its own cell, the
 // nodes that are nearer than grid_low of what it has, which from there are
-// few.
+// few.  With *odd set (nested_kernel) every cell is left undecided.
 __global__ void __launch_bounds__(256)
-grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out) {
+grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out,
+            const uint32_t *odd) {
     // pending inner nodes of a wave: children and squared distance
     __shared__ uint4 stack[4][kGridStack];
     const uint32_t w = threadIdx.x >> 6, b = blockIdx.x * 4u + w;
@@ -2691,6 +2727,14 @@ grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out) {
     const uint32_t lane = lane_id();
     const uint32_t by = (g.n[1] + 3u) / 4u, bz = (g.n[2] + 3u) / 4u;
     const uint32_t ix0 = b / bz / by * 4u, iy0 = b / bz % by * 4u, iz0 = b % bz * 4u;
+    const uint32_t ix = ix0 + (lane >> 4), iy = iy0 + ((lane >> 2) & 3u),
+                   iz = iz0 + (lane & 3u);
+    const bool mine = (ix < g.n[0]) & (iy < g.n[1]) & (iz < g.n[2]);
+    uint32_t *const cell = out + ((size_t)ix * g.n[1] + iy) * g.n[2] + iz;
+    if (*odd) {
+        if (mine) *cell = ballgrid::kNoBounds;
+        return;
+    }
     const f3 mid = f3{ballgrid::grid_centre(g, 0, ix0 + 2u),
                       ballgrid::grid_centre(g, 1, iy0 + 2u),
                       ballgrid::grid_centre(g, 2, iz0 + 2u)};
@@ -2765,8 +2809,6 @@ grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out) {
             sp = min(sp + (uint32_t)__popc(all), kGridStack);
         }
     }
-    const uint32_t ix = ix0 + (lane >> 4), iy = iy0 + ((lane >> 2) & 3u),
-                   iz = iz0 + (lane & 3u);
     const f3 c = f3{ballgrid::grid_centre(g, 0, ix), ballgrid::grid_centre(g, 1, iy),
                     ballgrid::grid_centre(g, 2, iz)};
     // squared: to the nearest voxel so far; and what need not be looked at
@@ -2784,9 +2826,7 @@ grid_kernel(Tree t, ballgrid::Grid g, uint32_t blocks, uint32_t *out) {
             node = nd.ref;
         }
     }
-    if ((ix < g.n[0]) & (iy < g.n[1]) & (iz < g.n[2]))
-        out[((size_t)ix * g.n[1] + iy) * g.n[2] + iz] =
-            ballgrid::grid_pack(g, low, best);
+    if (mine) *cell = ballgrid::grid_pack(g, low, best);
 }
 
 struct BallItem {
@@ -3566,8 +3606,13 @@ int upload(voxg_tree *t) {
         uint32_t *d = (uint32_t *)((char *)t->d_mem + tb.grid_off);
         const uint32_t blocks = (g.n[0] + 3) / 4 * ((g.n[1] + 3) / 4) *
                                 ((g.n[2] + 3) / 4);
+        const uint32_t nodes = (uint32_t)h.nodes.size();
+        HIPCHK(hipMemset(d + cells, 0, sizeof(uint32_t)));
+        hipLaunchKernelGGL(dev::nested_kernel, dim3((nodes + 255) / 256), dim3(256),
+                           0, nullptr, dev_tree(t), nodes, d + cells);
+        HIPCHK(hipGetLastError());
         hipLaunchKernelGGL(dev::grid_kernel, dim3((blocks + 3) / 4), dim3(256), 0,
-                           nullptr, dev_tree(t), g, blocks, d);
+                           nullptr, dev_tree(t), g, blocks, d, d + cells);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(nullptr));
         g.cells = d;
