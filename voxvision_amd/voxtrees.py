@@ -42,6 +42,15 @@ def _rows(x, stream):
     return t
 
 
+def _overlap(x, rows):
+    """Whether the contiguous tensor x shares memory with one of rows."""
+    def ends(t):
+        a = t.data_ptr()
+        return a, a + t.numel() * t.element_size()
+    a, b = ends(x)
+    return any(a < d and c < b for c, d in map(ends, rows))
+
+
 class Tree:
     """A flattened tree resident in device memory (immutable)."""
 
@@ -147,8 +156,10 @@ def make_tree(dots, voxel=(1.0, 1.0, 1.0)):
 def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
                           stream=None):
     """Batched vox_ray_tree_intersection.  o, d: (n, 3) arrays or tensors.
-    Returns (voxel_id uint32-as-int64 tensor, hit (3, n) float32 tensor
-    [, leaf node index tensor])."""
+    hit_init: a (3, n) tensor or three arrays of n floats that the hits are
+    written to (a missed ray's entries are left as they are); it may share
+    memory with o and d.  Returns (voxel_id uint32-as-int64 tensor, hit (3, n)
+    float32 tensor or hit_init [, leaf node index tensor])."""
     L = _lib.load()
     o = _rows(o, stream)
     d = _rows(d, stream)
@@ -164,8 +175,8 @@ def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
     if hit is None:
         hit = torch.empty((3, n), dtype=torch.float32, device="cuda")
     else:  # hits are written while other rays are read
-        o, d = (x.clone() if x.untyped_storage().data_ptr() ==
-                hit.untyped_storage().data_ptr() else x for x in (o, d))
+        rows = [hit[k][:n] for k in range(3)]
+        o, d = (x.clone() if _overlap(x, rows) else x for x in (o, d))
     check(L.voxg_ray_batch_rows(tree.handle, n, o.data_ptr(), d.data_ptr(),
                                 vox.data_ptr(),
                                 leaf.data_ptr() if want_leaf else None,
