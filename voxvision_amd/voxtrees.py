@@ -32,14 +32,33 @@ def _dev_f32(x, n=None, cols=None):
     return t
 
 
-def _rows(x, stream):
-    """x as n rows of three floats on the device.  A call on another stream
-    than the current one reads a copy: the caller may go on writing x."""
-    t = _dev_f32(x).reshape(-1, 3)
-    if stream is not None and \
-            stream.cuda_stream != torch.cuda.current_stream().cuda_stream:
-        t = t.clone()
-    return t
+def _other(stream):
+    """`stream` if it is another one than the current stream, else None."""
+    if stream is None or \
+            stream.cuda_stream == torch.cuda.current_stream().cuda_stream:
+        return None
+    return stream if isinstance(stream, torch.cuda.Stream) else \
+        torch.cuda.ExternalStream(stream.cuda_stream)
+
+
+def _hand_over(stream, *tensors):
+    """Before a launch on `stream` (from _other; None: nothing to do) that
+    uses tensors written on, or allocated for, the current stream: the launch
+    waits for the current stream's work so far, and a tensor that is dropped
+    is not handed out again until `stream` is done with it."""
+    if stream is not None:
+        stream.wait_stream(torch.cuda.current_stream())
+        for t in tensors:
+            if t is not None:
+                t.record_stream(stream)
+
+
+def _input(x, stream, rows=False):
+    """x as device floats, one row of them or, with `rows`, n rows of three.
+    A call on another stream reads a copy: the caller may go on writing x on
+    the current stream."""
+    t = _dev_f32(x).reshape((-1, 3) if rows else -1)
+    return t if stream is None else t.clone()
 
 
 def _overlap(x, rows):
@@ -158,11 +177,15 @@ def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
     """Batched vox_ray_tree_intersection.  o, d: (n, 3) arrays or tensors.
     hit_init: a (3, n) tensor or three arrays of n floats that the hits are
     written to (a missed ray's entries are left as they are); it may share
-    memory with o and d.  Returns (voxel_id uint32-as-int64 tensor, hit (3, n)
+    memory with o and d.  With `stream` another one than the current stream
+    the rays are those that the current stream holds at this point (the work
+    on `stream` waits for it), and the results are there once `stream` has
+    reached them.  Returns (voxel_id uint32-as-int64 tensor, hit (3, n)
     float32 tensor or hit_init [, leaf node index tensor])."""
     L = _lib.load()
-    o = _rows(o, stream)
-    d = _rows(d, stream)
+    other = _other(stream)
+    o = _input(o, other, rows=True)
+    d = _input(d, other, rows=True)
     n = o.shape[0]
     if d.shape[0] < n:
         raise ValueError("a direction for every origin")
@@ -177,6 +200,7 @@ def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
     else:  # hits are written while other rays are read
         rows = [hit[k][:n] for k in range(3)]
         o, d = (x.clone() if _overlap(x, rows) else x for x in (o, d))
+    _hand_over(other, o, d, vox, leaf, hit[0], hit[1], hit[2])
     check(L.voxg_ray_batch_rows(tree.handle, n, o.data_ptr(), d.data_ptr(),
                                 vox.data_ptr(),
                                 leaf.data_ptr() if want_leaf else None,
@@ -205,14 +229,17 @@ def ray_counts(tree, o, d, stream=None):
 
 
 def tree_ball_collidep(tree, c, r, stream=None):
-    """Batched vox_tree_ball_collidep: (n,3) centres, (n,) radii -> uint8."""
+    """Batched vox_tree_ball_collidep: (n,3) centres, (n,) radii -> uint8.
+    `stream` as in ray_tree_intersection."""
     L = _lib.load()
-    c = _rows(c, stream)
-    r = _dev_f32(r).reshape(-1)
+    other = _other(stream)
+    c = _input(c, other, rows=True)
+    r = _input(r, other)
     n = c.shape[0]
     if r.shape[0] < n:
         raise ValueError("a radius for every centre")
     out = torch.empty(n, dtype=torch.uint8, device="cuda")
+    _hand_over(other, c, r, out)
     check(L.voxg_ball_batch_rows(tree.handle, n, c.data_ptr(), r.data_ptr(),
                                  out.data_ptr(), _stream(stream)),
           "voxg_ball_batch_rows")
