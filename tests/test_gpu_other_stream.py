@@ -1,4 +1,4 @@
-"""Ray and ball calls with `stream` naming another stream than the current
+"""Ray, ball, count and selection calls with `stream` naming another stream than the current
 one: the inputs are written on the current stream behind queued work and
 overwritten right after the call, the call's temporaries are dropped and
 their memory asked for again while the other stream is still busy, and the
@@ -73,3 +73,43 @@ def test_another_stream(gpu, n, busy, plain):
     assert _same(b, kept)
     assert torch.equal(c, balls)
     del again
+
+
+@pytest.mark.parametrize("busy", ["current", "other"])
+def test_counts_and_selection_on_another_stream(gpu, busy):
+    VT, tree, o, d, r = _scene(5000)
+    dim = (96, 80, 64)
+    raw = (torch.arange(96 * 80 * 64, device="cuda") * 37 % 251).to(torch.uint8)
+    want = (VT.ray_counts(tree, o, d), VT.ball_counts(tree, o, r),
+            VT.raw_select(raw, dim, 1, threshold=200))
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        VT.ray_counts(tree, o, d)
+        VT.raw_select(raw, dim, 1, threshold=200)
+    big = torch.zeros(1 << 26, device="cuda")
+    ins = [torch.full_like(x, float("nan")) for x in (o, d, r)]
+    src = torch.zeros_like(raw)
+    torch.cuda.synchronize()
+    for k in range(3):
+        if busy == "current":
+            _busy(big)
+        else:
+            with torch.cuda.stream(side):
+                _busy(big)
+        if k == 0:
+            ins[0].copy_(o)
+            ins[1].copy_(d)
+            got = VT.ray_counts(tree, ins[0], ins[1], stream=side)
+        elif k == 1:
+            ins[2].copy_(r)
+            got = VT.ball_counts(tree, ins[0], ins[2], stream=side)
+        else:
+            src.copy_(raw)
+            got = VT.raw_select(src, dim, 1, threshold=200, stream=side)
+            again = [torch.full_like(got, -1.0) for _ in range(4)]
+            side.synchronize()
+            assert torch.equal(got, want[k])
+            del again
+        if k < 2:
+            assert got == want[k]
+        torch.cuda.synchronize()

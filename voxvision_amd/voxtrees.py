@@ -219,6 +219,7 @@ def ray_counts(tree, o, d, stream=None):
     o = _dev_f32(o).reshape(-1, 3).t().contiguous()
     d = _dev_f32(d).reshape(-1, 3).t().contiguous()
     c = _lib.Counts()
+    _hand_over(_other(stream), o, d)
     check(L.voxg_ray_batch_count(tree.handle, o.shape[1], o[0].data_ptr(),
                                  o[1].data_ptr(), o[2].data_ptr(),
                                  d[0].data_ptr(), d[1].data_ptr(),
@@ -251,6 +252,7 @@ def ball_counts(tree, c, r, stream=None):
     c = _dev_f32(c).reshape(-1, 3).t().contiguous()
     r = _dev_f32(r).reshape(-1).contiguous()
     cnt = _lib.Counts()
+    _hand_over(_other(stream), c, r)
     check(L.voxg_ball_batch_count(tree.handle, c.shape[1], c[0].data_ptr(),
                                   c[1].data_ptr(), c[2].data_ptr(),
                                   r.data_ptr(), C.byref(cnt),
@@ -289,12 +291,17 @@ def raw_select(samples, dim, samplesize, lo=None, hi=None, threshold=None,
     work = torch.empty(nb, dtype=torch.uint8, device="cuda")
     cnt = torch.empty(1, dtype=torch.int64, device="cuda")
     st = _stream(stream)
+    other = _other(stream)
+    _hand_over(other, work, cnt)
     check(L.voxg_raw_count(samples.data_ptr(), d, samplesize, lo, hi,
                            work.data_ptr(), cnt.data_ptr(), st),
           "voxg_raw_count")
+    if other is not None:
+        other.synchronize()
     m = int(cnt.item())
     xyz = torch.empty((m, 3), dtype=torch.float32, device="cuda")
     if m:
+        _hand_over(other, xyz)
         check(L.voxg_raw_write(d, v, work.data_ptr(), xyz.data_ptr(), m, st),
               "voxg_raw_write")
     return xyz
