@@ -90,7 +90,7 @@ typedef struct {
     uint32_t depth;          /* levels, root = 1 */
     uint32_t stack_entries;  /* traversal stack bound: one entry per
                                 inner level, depth-1 (at least 1) */
-    uint64_t device_bytes;   /* flattened tree and ball grid in HBM */
+    uint64_t device_bytes;   /* flattened tree size in HBM */
     float bbox_min[3], bbox_max[3];
     float voxel[3];          /* voxel size snapshot taken at build/upload */
 } voxg_tree_info;
@@ -187,6 +187,13 @@ int voxg_ball_batch(const voxg_tree *tree, size_t n, const float *cx,
 /* voxg_ball_batch over centres stored as n rows of three floats. */
 int voxg_ball_batch_rows(const voxg_tree *tree, size_t n, const float *c,
                          const float *r, uint8_t *out, hipStream_t stream);
+/* Bounds on a grid over the tree's box answer most ball queries (at most 32
+ * bytes of HBM per node and 8.4 MB).  The tree makes them by itself ahead of the
+ * call whose queries, with those before, are worth it, never under stream
+ * capture; results are the same without.  This makes them now and returns
+ * when they are there, for programs that capture ball calls before they have
+ * made many (VOXG_EINVAL if `stream` is being captured). */
+int voxg_tree_prepare_balls(const voxg_tree *tree, hipStream_t stream);
 
 /* Editable host trees (vox_insert_voxel / vox_delete_voxel,
  * src/voxtrees/tree.h:96,114, tree.c:437-835).  The tree lives in host

@@ -1,0 +1,213 @@
+"""When a tree makes its ball grid, and that answers are the same before and
+after: on request, by enough queries, by many small launches, by two threads
+on two streams at once, not under stream capture, and not for trees that have
+none; a tree takes no memory for it until then."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(oracle, kind="blobs", voxel=(1.0, 1.0, 1.0), n=5000, seed=3):
+    """Centres in the box and around it, radii from a voxel to the box."""
+    from voxvision_amd import scenes, voxtrees as VT
+    vol = scenes.blobs64(seed) if kind == "blobs" else \
+        scenes.shell_volume(150, 0.02)
+    dots = scenes.volume_to_dots(vol)[:, :3] * np.array(voxel, np.float32)
+    rng = np.random.default_rng(seed)
+    lo, hi = dots.min(0) - 3.0, dots.max(0) + 4.0
+    c = rng.uniform(lo, hi, (n, 3)).astype(np.float32)
+    r = np.exp(rng.uniform(np.log(0.3), np.log(0.3 * (hi - lo).max()),
+                           n)).astype(np.float32)
+    want = torch.from_numpy(oracle.Tree(dots, voxel).balls(c, r)).cuda()
+    assert 0 < int(want.sum()) < n
+    return (VT, VT.make_tree(dots, voxel), torch.from_numpy(c).cuda(),
+            torch.from_numpy(r).cuda(), want)
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+@pytest.mark.parametrize("kind", ["blobs", "shell"])
+@pytest.mark.parametrize("voxel", [(1.0, 1.0, 1.0), (0.5, 0.75, 3.0)])
+def test_on_request(gpu, oracle, kind, voxel):
+    VT, G, c, r, want = _scene(oracle, kind, voxel)
+    assert torch.equal(VT.tree_ball_collidep(G, c, r), want)
+    G.prepare_balls()
+    G.prepare_balls()
+    assert torch.equal(VT.tree_ball_collidep(G, c, r), want)
+
+
+@pytest.mark.parametrize("n,calls", [(4 << 20, 2), (5000, 60)])
+def test_by_queries(gpu, oracle, n, calls):
+    """Past the line (2^21 queries, 7/2 a cell, 2^16 a launch) either way."""
+    VT, G, c, r, want = _scene(oracle)
+    i = torch.arange(n, device="cuda") % len(want)
+    ci, ri, wi = c[i], r[i], want[i]
+    for _ in range(calls):
+        assert torch.equal(VT.tree_ball_collidep(G, ci, ri), wi)
+
+
+def test_bodies_and_the_tree_alone(gpu, oracle):
+    from voxvision_amd import voxrnd
+    VT, G, c, r, want = _scene(oracle)
+    for k in range(2):
+        pos = [c[:, j].contiguous() for j in range(3)]
+        last = [x + 1.0 for x in pos]
+        hit = voxrnd.cd_collide(G, pos, last, r)
+        assert torch.equal(hit, want)
+        G.prepare_balls()
+
+
+def test_two_threads_two_streams(gpu, oracle):
+    VT, G, c, r, want = _scene(oracle)
+    n = 4 << 20  # the first launch makes the grid
+    i = torch.arange(n, device="cuda") % len(want)
+    ci, ri, wi = c[i], r[i], want[i]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for s in streams:
+        with torch.cuda.stream(s):
+            VT.tree_ball_collidep(G, c[:1], r[:1])
+    torch.cuda.synchronize()
+    got = [None] * 2
+    gate = threading.Barrier(2)
+
+    def ask(k):
+        with torch.cuda.stream(streams[k]):
+            gate.wait()
+            got[k] = [VT.tree_ball_collidep(G, ci, ri) for _ in range(3)]
+            streams[k].synchronize()
+    th = [threading.Thread(target=ask, args=(k,)) for k in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for out in got:
+        for x in out:
+            assert torch.equal(x, wi)
+
+
+@pytest.mark.parametrize("before", ["none", "asked", "prepared"])
+def test_capture(gpu, oracle, before):
+    """A captured call, however large, replays right, whether the grid was
+    there before the capture, is made between replays, or never."""
+    VT, G, c, r, want = _scene(oracle)
+    n = 4 << 20
+    i = torch.arange(n, device="cuda") % len(want)
+    ci, ri, wi = c[i], r[i], want[i]
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        VT.tree_ball_collidep(G, c, r)  # the stream's workspace
+        if before == "asked":
+            VT.tree_ball_collidep(G, ci, ri)
+        elif before == "prepared":
+            G.prepare_balls()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        out = VT.tree_ball_collidep(G, ci, ri)
+    for k in range(3):
+        out.fill_(7)
+        g.replay()
+        assert torch.equal(out, wi)
+        assert torch.equal(VT.tree_ball_collidep(G, ci, ri), wi)
+
+
+def test_prepare_under_capture_is_refused(gpu, oracle):
+    VT, G, c, r, want = _scene(oracle)
+    from voxvision_amd import _lib
+    s = torch.cuda.Stream()
+    x = torch.zeros(4, device="cuda")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        x.add_(1.0)
+        rc = _lib.load().voxg_tree_prepare_balls(G.handle, s.cuda_stream)
+    assert rc == -22
+    g.replay()
+    G.prepare_balls()
+    assert torch.equal(VT.tree_ball_collidep(G, c, r), want)
+
+
+def test_queries_while_another_thread_captures(gpu, oracle):
+    """The stream of a tree's first queries is being captured while another
+    thread's queries make the grid and ask whether it is there."""
+    VT, G, c, r, want = _scene(oracle)
+    n = 4 << 20
+    i = torch.arange(n, device="cuda") % len(want)
+    ci, ri, wi = c[i], r[i], want[i]
+    s, side = torch.cuda.Stream(), torch.cuda.Stream()
+    for st in (s, side):
+        with torch.cuda.stream(st):
+            VT.tree_ball_collidep(G, c, r)
+    torch.cuda.synchronize()
+    x = torch.zeros(4, device="cuda")
+    outs = [torch.empty(n, dtype=torch.uint8, device="cuda")
+            for _ in range(4)]
+    cols = [ci[:, k].contiguous() for k in range(3)]
+    from voxvision_amd import _lib
+    L = _lib.load()
+    errors = []
+
+    def ask():  # (the library alone: torch's allocator is captured)
+        _lib.check(L.voxg_init(0))
+        for out in outs:
+            errors.append(L.voxg_ball_batch(
+                G.handle, n, *[t.data_ptr() for t in cols], ri.data_ptr(),
+                out.data_ptr(), side.cuda_stream))
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+        x.add_(1.0)
+        th = threading.Thread(target=ask)
+        th.start()
+        th.join()
+        x.add_(1.0)
+    assert errors == [0] * 4
+    side.synchronize()
+    for out in outs:
+        assert torch.equal(out, wi)
+    for k in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert x.tolist() == [2.0 * (k + 1)] * 4
+
+
+@pytest.mark.parametrize("dots", [[], [[3, 4, 5]],
+                                  [[3, 4, 5], [4, 4, 5], [9, 4, 5]]])
+def test_trees_without_one(gpu, oracle, dots):
+    from voxvision_amd import voxtrees as VT
+    d = np.array(dots, np.float32).reshape(-1, 3)
+    G = VT.make_tree(d)
+    rng = np.random.default_rng(1)
+    c = rng.uniform(0, 12, (300, 3)).astype(np.float32)
+    r = rng.uniform(0.1, 4, 300).astype(np.float32)
+    want = oracle.Tree(d).balls(c, r)
+    for _ in range(2):
+        got = VT.tree_ball_collidep(G, c, r).cpu().numpy()
+        assert np.array_equal(got, want)
+        G.prepare_balls()
+
+
+def test_memory(gpu, oracle):
+    """The tree alone takes what its info and the plan say; the grid comes
+    and goes with the tree that made one."""
+    from voxvision_amd import scenes, voxtrees as VT
+    occ = np.random.default_rng(5).random((128, 128, 128)) < 0.2
+    dots = scenes.volume_to_dots(occ)
+    plan, _ = VT.plan(dots)
+    trees = [VT.make_tree(dots) for _ in range(2)]
+    del trees
+    free0 = _free()
+    G = VT.make_tree(dots)
+    assert G.info["device_bytes"] == plan["device_bytes"]
+    bare = free0 - _free()
+    assert bare <= plan["device_bytes"] + (4 << 20)
+    G.prepare_balls()
+    G.release()
+    assert _free() >= free0 - (4 << 20)

@@ -53,3 +53,4 @@ def test_boxes_that_hold_less(gpu, oracle, what):
     for _ in range(3):
         got = VT.tree_ball_collidep(G, ct, rt)
         assert np.array_equal(got.cpu().numpy(), want)
+        G.prepare_balls()

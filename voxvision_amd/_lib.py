@@ -38,6 +38,7 @@ EXPORTS = [
     "voxg_synchronize", "voxg_release_stream", "voxg_test_fail_at",
     "voxg_test_stack_bound", "voxg_test_server_hold", "voxg_test_plan_cut",
     "voxg_ray_batch_noalloc", "voxg_ray_batch_rows", "voxg_ball_batch_rows",
+    "voxg_tree_prepare_balls",
     "voxg_lights_create", "voxg_lights_release", "voxg_lights_set_ambient",
     "voxg_lights_insert", "voxg_lights_delete", "voxg_lights_clear",
     "voxg_lights_count", "voxg_lights_get",
@@ -128,6 +129,7 @@ def load():
         C.POINTER(Counts), P]
     L.voxg_ball_batch.argtypes = [P, S, P, P, P, P, P, P]
     L.voxg_ball_batch_rows.argtypes = [P, S, P, P, P, P]
+    L.voxg_tree_prepare_balls.argtypes = [P, P]
     L.voxg_ball_batch_count.argtypes = [P, S, P, P, P, P,
                                         C.POINTER(Counts), P]
     L.voxg_camera_set_window_size.argtypes = [C.POINTER(Camera), I, I]

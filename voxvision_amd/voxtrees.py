@@ -134,6 +134,14 @@ class Tree:
             "voxg_tree_voxel_coords")
         return out
 
+    def prepare_balls(self, stream=None):
+        """Make the bounds that answer most ball queries now, as a tree
+        otherwise does once it has had enough of them (outside stream
+        capture); results are the same without."""
+        check(_lib.load().voxg_tree_prepare_balls(self.handle,
+                                                  _stream(stream)),
+              "voxg_tree_prepare_balls")
+
     def node_ptr(self, idx):
         return _lib.load().voxg_tree_node_ptr(self.handle, int(idx))
 
