@@ -304,7 +304,8 @@ struct Loc {
 struct Tally {
     uint64_t inner = 0, leaves = 0, dense = 0, overflow = 0;
     uint64_t ndots = 0, dense_ids = 0;
-    bool too_big = false;
+    bool too_big = false, inverted = false;
+    int32_t largest = 0;  // magnitude_bits
     void add(const Tally &o) {
         inner += o.inner;
         leaves += o.leaves;
@@ -313,6 +314,8 @@ struct Tally {
         ndots += o.ndots;
         dense_ids += o.dense_ids;
         too_big |= o.too_big;
+        inverted |= o.inverted;
+        largest = std::max(largest, o.largest);
     }
 };
 
@@ -322,9 +325,13 @@ Loc<typename View::N> record(const View &view, typename View::N n,
                              const float V[3], Tally &t) {
     Loc<typename View::N> l;
     std::memset(&l.r, 0, sizeof(l.r));
+    int32_t largest = t.largest;
     for (int k = 0; k < 3; k++) {
         l.r.bmin[k] = View::bmin(n)[k];
         l.r.bmax[k] = View::bmax(n)[k];
+        largest = std::max({largest, magnitude_bits(l.r.bmin[k]),
+                            magnitude_bits(l.r.bmax[k])});
+        t.inverted |= !(l.r.bmin[k] <= l.r.bmax[k]);
     }
     const uint32_t f = View::flags(n);
     l.r.info = f & (NT_TYPE_MASK | NT_OVERFLOW);
@@ -334,7 +341,10 @@ Loc<typename View::N> record(const View &view, typename View::N n,
     l.src = View::src(n);
     l.dots = nullptr;
     if ((f & NT_TYPE_MASK) == NT_INNER) {
-        for (int k = 0; k < 3; k++) l.r.c[k] = View::center(n)[k];
+        for (int k = 0; k < 3; k++) {
+            l.r.c[k] = View::center(n)[k];
+            largest = std::max(largest, magnitude_bits(l.r.c[k]));
+        }
         uint32_t mask = 0;
         for (int c = 0; c < 8; c++)
             if (!View::null(View::child(n, c))) mask |= 1u << c;
@@ -354,6 +364,7 @@ Loc<typename View::N> record(const View &view, typename View::N n,
         t.dense_ids += (uint64_t)dim[0] * dim[1] * dim[2];
         t.dense++;
     }
+    t.largest = largest;
     return l;
 }
 
@@ -529,6 +540,8 @@ int flatten(const View &view, typename View::N root, const float V[3],
     //    over the records (children are [ref, ref + popcount)); dots first,
     //    then dense voxels.  The leaves' dots are copied afterwards, on the
     //    pool (each leaf's source is a cache miss of its own)
+    for (int l = 0; l < 3; l++)
+        tally.largest = std::max(tally.largest, magnitude_bits(V[l]));
     const uint64_t ndots = tally.ndots;
     out.dots.resize(3 * ndots);
     uint64_t dot_next = 0, dense_next = ndots;
@@ -561,7 +574,9 @@ int flatten(const View &view, typename View::N root, const float V[3],
         const unsigned nt = (unsigned)std::min<size_t>(
             std::min(hw, kMaxThreads), (leaves.size() + chunk - 1) / chunk);
         std::atomic<size_t> next_leaf{0};
+        std::mutex mu;
         auto work = [&](unsigned) {
+            int32_t largest = 0;
             for (;;) {
                 const size_t b = next_leaf.fetch_add(chunk);
                 if (b >= leaves.size()) break;
@@ -572,15 +587,21 @@ int flatten(const View &view, typename View::N root, const float V[3],
                     const float *p = dots[leaves[j]];
                     float *q = out.dots.data() + 3 * (size_t)r.ref;
                     for (uint32_t k = 0; k < cnt; k++) {
-                        q[3 * k + 0] = p[4 * k + 0];
-                        q[3 * k + 1] = p[4 * k + 1];
-                        q[3 * k + 2] = p[4 * k + 2];
+                        for (int l = 0; l < 3; l++) {
+                            q[3 * k + l] = p[4 * k + l];
+                            largest = std::max(largest,
+                                               magnitude_bits(p[4 * k + l]));
+                        }
                     }
                 }
             }
+            std::lock_guard<std::mutex> g(mu);
+            tally.largest = std::max(tally.largest, largest);
         };
         run_pool(nt, work);
     }
+    out.largest = tally.largest;
+    out.inverted = tally.inverted;
     out.ndots = ndots;
     out.voxel_ids = ndots + tally.dense_ids;
     return 0;

@@ -2,6 +2,7 @@
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <string>
 #include <vector>
@@ -20,7 +21,23 @@ struct HostTree {
     uint64_t inner = 0, leaves = 0, dense = 0, overflow = 0;
     uint32_t depth = 0;
     float voxel[3] = {1.0f, 1.0f, 1.0f};
+    int32_t largest = 0;    // magnitude_bits of the largest coordinate
+    bool inverted = false;  // a box with a NaN corner or max below min
 };
+
+// A float's magnitude as an integer: the order of the magnitudes, infinities
+// and NaN above them all.
+inline int32_t magnitude_bits(float x) {
+    int32_t w;
+    memcpy(&w, &x, sizeof(w));
+    return w & 0x7fffffff;
+}
+
+// Whether the tests of raymath.h hold for the tree: its boxes, centres and
+// voxels finite, at most 2^60 in magnitude and not inverted.
+inline bool plain(const HostTree &h) {
+    return h.largest <= 0x5d800000 && !h.inverted;
+}
 
 int build_tree(const float *xyz, size_t n, size_t stride, const float V[3],
                HostTree &out, std::string &err);

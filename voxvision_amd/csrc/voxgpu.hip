@@ -105,40 +105,6 @@ static std::vector<float> cut_of(const HostTree &h) {
     return out;
 }
 
-// Whether the tests of raymath.h hold for the tree: its boxes, centres and
-// voxels finite, at most 2^60 in magnitude and not inverted.  The largest
-// magnitude is taken over the words' bits, which order as the floats do and
-// put infinities and NaN above them all (a dense leaf's dimensions, where
-// others have a centre, are far below): vector code, 2.6 times as fast as a
-// test per coordinate, which took 0.58 of an upload's 1.8 ms for the 233,000
-// nodes of a 256^3 scene.
-static bool plain_tree(const HostTree &h) {
-    constexpr int32_t kLimit = 0x5d800000;  // 2^60
-    auto up = [](int32_t &top, int32_t w) {
-        w &= 0x7fffffff;
-        top = w > top ? w : top;
-    };
-    static_assert(offsetof(NodeRec, bmax) == 12 && offsetof(NodeRec, c) == 32,
-                  "words 0 to 5 and 8 to 10 of a record are coordinates");
-    int32_t top[12] = {0}, inverted = 0;
-    for (const NodeRec &n : h.nodes) {
-        int32_t w[12];
-        std::memcpy(w, &n, sizeof(w));
-        for (int k = 0; k < 12; k++) up(top[k], w[k]);
-        for (int k = 0; k < 3; k++) inverted |= !(n.bmin[k] <= n.bmax[k]);
-    }
-    int32_t most = 0;
-    for (int k : {0, 1, 2, 3, 4, 5, 8, 9, 10}) up(most, top[k]);
-    auto bits = [](float x) {
-        int32_t w;
-        std::memcpy(&w, &x, 4);
-        return w;
-    };
-    for (float x : h.dots) up(most, bits(x));
-    for (float x : h.voxel) up(most, bits(x));
-    return most <= kLimit && !inverted;
-}
-
 // The shape of a tree's ball grid (ball_grid.h); false: none.
 static bool grid_of(const HostTree &h, bool plain, ballgrid::Grid &g) {
     std::memset(&g, 0, sizeof(g));
@@ -3725,7 +3691,7 @@ int upload(voxg_tree *t) {
 
 int finish_tree(voxg_tree *t, voxg_tree **out) {
     t->stack_bound = stack_bound_of(t->host);
-    t->odd = !plain_tree(t->host);
+    t->odd = !plain(t->host);
     if (!grid_of(t->host, !t->odd, t->balls.grid)) t->balls.none = true;
     int rc = upload(t);
     if (rc) {
