@@ -43,9 +43,9 @@ def test_on_request(gpu, oracle, kind, voxel):
     assert torch.equal(VT.tree_ball_collidep(G, c, r), want)
 
 
-@pytest.mark.parametrize("n,calls", [(4 << 20, 2), (5000, 60)])
+@pytest.mark.parametrize("n,calls", [(4 << 20, 2), (5000, 80)])
 def test_by_queries(gpu, oracle, n, calls):
-    """Past the line (2^21 queries, 7/2 a cell, 2^16 a launch) either way."""
+    """Past the line (2^21 queries, 7/2 a cell, 2^15 a launch) either way."""
     VT, G, c, r, want = _scene(oracle)
     i = torch.arange(n, device="cuda") % len(want)
     ci, ri, wi = c[i], r[i], want[i]

@@ -5,19 +5,21 @@
 // is a depth-first search over (node, origin) pairs in a fixed order:
 // the child holding the entry point first, then the children behind the
 // dividing planes in L1-distance order.  Each lane keeps the pair it is
-// working on in registers and the pending pairs on a stack.  Plane points
-// depend only on the node and its entry point, so they are computed when
-// the node is visited and pushed (last-visited first); the visit order,
-// every origin and every rounding step are the reference's, which makes
-// the results bit-identical.  The stack is a ring of K entries per lane in
+// working on in registers and the pending pairs on a stack, one entry per
+// node: its index, its entry point and the planes whose children are still
+// to come.  A plane point depends only on the node and its entry point and is
+// computed again when its child's turn comes; the visit order, every origin
+// and every rounding step are the reference's, which makes the results
+// bit-identical.  The stack is a ring of K entries per lane in
 // LDS; older entries spill to an HBM buffer and come back when the ring
 // empties, so any depth stays exact.
 //
-// Work distribution: persistent waves.  A wave keeps 64 rays in flight and
-// refills idle lanes from a global ray counter (one atomic per refill,
-// lanes numbered with a ballot and mbcnt), so long rays do not hold a whole
-// wave.  The counter resets itself when the last wave leaves, so a launch
-// needs no memset and can be captured in a graph.
+// Work distribution: persistent waves.  A wave keeps up to 64 rays in flight
+// and refills idle lanes (numbered with a ballot and mbcnt) from a pool of
+// units, so long rays do not hold a whole wave.  The first pools are shares by
+// the wave's place in the grid, the others come from one counter per XCD.  The
+// last wave to leave clears the counters, so a launch needs no memset and can
+// be captured in a graph.
 //
 // Floating point: compiled with -ffp-contract=off; __builtin_fmaf marks the
 // reference's fused sites (geom-sse.c:109,135; simple-camera.c:29;
@@ -633,14 +635,14 @@ constexpr size_t kCounterBytes =
 // waiting for a wave-wide refill.
 template <class Src, class Sink>
 struct ChunkWork {
-    // 8 waves per SIMD (at most 64 VGPRs; it takes 54)
+    // 8 waves per SIMD (at most 64 VGPRs)
     static constexpr int kMinWavesPerSimd = 8;
     static constexpr uint32_t kPool = 4, kFew = 0;
     static constexpr int kSpread = 16;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
     // XCD hand-out: one contiguous range of the units per XCD
     __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
-        Src src;
+    Src src;
     Sink sink;
     uint32_t n, chunk;
     __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &) const {
@@ -692,7 +694,7 @@ struct MultiWork {
     static constexpr int kSpread = 16;
     __host__ __device__ __forceinline__ bool keeps_queue() const { return true; }
     __device__ __forceinline__ uint32_t xcd_shift() const { return 0; }
-        Src src;
+    Src src;
     Sink sink;
     const BatchItem *items;
     uint32_t n_items, chunk;
@@ -873,7 +875,8 @@ struct RenderItem {
 template <bool MULTI>
 struct BlockWork {
     // 6 waves per SIMD (at most 80 VGPRs) fit without spilling for one
-    // render; the multi-job form would spill at that floor
+    // render, which then takes 70; the multi-job form takes 86 (5 waves) and
+    // would spill at that floor
     static constexpr int kMinWavesPerSimd = MULTI ? 1 : 6;
     static constexpr uint32_t kPool = 1, kFew = 0;
     static constexpr int kSpread = 8;
@@ -894,7 +897,7 @@ struct BlockWork {
         if constexpr (MULTI) return 0;
         else return group;
     }
-        uint32_t units_per_block_host() const { return 1u; }
+    uint32_t units_per_block_host() const { return 1u; }
     // reads once per thread what the block pre-pass counted on the device;
     // returns the number of units
     __device__ __forceinline__ uint32_t prepare(uint32_t n, uint32_t &qf) const {
@@ -1773,7 +1776,7 @@ block_cull_kernel(RenderItem it, uint32_t npix, Ctrl *ctrl,
     // (not when counting: the counts add one root box test per finished
     // ray, which a deeper test would not match)
     const bool deep = !COUNT && it.t.ncut != 0;
-    // one thread per block, 4 blocks per thread
+    // one thread per block, kEach blocks per thread
     for (uint32_t j = 0; j < kEach; ++j) {
         const uint32_t lb = j * 256 + tid;
         const uint32_t blk = (tile0 >> 4) + lb;
@@ -3622,14 +3625,15 @@ void make_ball_grid(const voxg_tree *t) {
 // The grid is made ahead of the launch whose queries, with those before, are
 // worth it: not with the tree, since trees that are only traced, and those
 // that are edited again after a few queries, would pay for nothing (a commit
-// of an edited 256^3 scene 5.5 -> 6.3 ms, its tree 12.8 -> 20.1 MB).  Measured
-// on scenes of 64^3 to 256^3, it saves 0.08 ns a query (4 M: 523 us without,
-// 176 with) and 5 us a launch, however small (10,000: 20 and 13 us); it takes
-// 170 us, most of them the allocation, and 0.28 ns a cell (0.75 ms for 256^3).
-// In queries: a launch counts for 2^16 more than it has, against 2^21 and 7/2
-// a cell.  A tree that stops right after its grid was made then has lost
-// about as much as it could have gained.
-constexpr uint64_t kBallLaunch = 1u << 16, kBallGridBase = 1u << 21;
+// of an edited 256^3 scene 5.0 -> 6.1 ms, its tree 12.8 -> 20.1 MB).  Measured
+// on scenes of 53^3 to 256^3, it saves 0.03 to 0.1 ns a query, most often 0.08
+// (4 M of radii 0.5 to 8 in a 256^3 one: 525 us without, 178 with), and 1 to 3
+// us a launch, however small; it takes 170 us, most of them the allocation,
+// and 0.28 ns a cell (0.75 ms for 256^3).  In queries of 0.08 ns: a launch
+// counts for 2^15 more than it has, against 2^21 and 7/2 a cell.  A tree that
+// stops right after its grid was made then has lost about as much as it could
+// have gained.
+constexpr uint64_t kBallLaunch = 1u << 15, kBallGridBase = 1u << 21;
 
 ballgrid::Grid ball_grid_for(const voxg_tree *t, size_t n, hipStream_t stream) {
     BallGrid &b = t->balls;
@@ -5016,11 +5020,13 @@ bool srv_stream_overflow(voxg_server *s, int i) {
 // frame's pixels over the whole device, one launch sequence per frame.
 // Only when a group holds at least kSrvShareMin frames smaller than
 // kSrvSmallPixels do those share one multi-job launch of one 4x4 block
-// per lane (a lane then walks 16 pixels in turn, about 2 ms for a
-// 320x240 frame, but one launch serves them all): under load that keeps
-// the throughput 10% higher, while alone a small frame takes 0.6 ms
-// through the render path (a Poisson stream of 1000 requests/s: p99
-// 1.9 ms against 4.6 ms when every small frame took the shared launch).
+// per lane (a lane then walks 16 pixels in turn, about 1 ms, but one launch
+// serves them all).  A 320x240 or 640x480 frame of a 256^3 scene alone takes
+// 0.17 to 0.24 ms, submission to results, through the render path.  Frames
+// that come at once, BEST and ADAPTIVE, shared against one after the other:
+// 8 of 320x240 1.1 and 1.5 against 1.1 and 1.25 ms, 12 of them 1.2 and 1.5
+// against 1.5 and 1.9, 24 1.5 and 1.9 against 3.1 and 3.6; 8 of 640x480 1.5
+// and 1.7 against 1.3 and 1.6, 24 2.2 and 2.4 against 3.8 and 4.6.
 constexpr size_t kSrvSmallPixels = (size_t)1 << 19;
 constexpr size_t kSrvShareMin = 8;
 
@@ -5332,6 +5338,7 @@ int voxg_server_create(const voxg_server_config *cfg, voxg_server **out) {
     if (s->cfg.streams > 16) return fail(VOXG_EINVAL, "at most 16 streams");
     std::memset(&s->st, 0, sizeof(s->st));
     HIPCHK(hipGetDevice(&s->device));
+    (void)own_stream();  // its first use is not to fall into a request
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     size_t budget = s->cfg.hbm_budget ? s->cfg.hbm_budget : fr / 2;
