@@ -17,6 +17,7 @@
 #include <string>
 
 #include "../../include/voxgpu.h"
+#include "fastdiv.h"
 #include "voxg_internal.h"
 
 using voxg_internal::fail;
@@ -230,32 +231,9 @@ raw_total_kernel(RawWork w, uint32_t ntiles, uint32_t ngroups,
     }
 }
 
-// Division of 32-bit numbers by an invariant d >= 1 (Granlund and Montgomery
-// 1994, figure 4.1): exact for every dividend, 5 instructions instead of
-// the 35 of a 32-bit division.
-struct Divisor {
-    uint32_t d, mul, s1, s2;
-};
-
-Divisor divisor(uint32_t d) {
-    uint32_t l = 0;
-    while (l < 32 && (1ull << l) < d) l++;
-    Divisor v;
-    v.d = d;
-    v.mul = (uint32_t)((((1ull << l) - d) << 32) / d + 1);
-    v.s1 = l < 1 ? l : 1;
-    v.s2 = l > 1 ? l - 1 : 0;
-    return v;
-}
-
-__device__ __forceinline__ uint32_t quotient_of(uint32_t n, const Divisor &v) {
-    const uint32_t t = __umulhi(v.mul, n);
-    return (t + ((n - t) >> v.s1)) >> v.s2;
-}
-
 struct RawOut {
     uint64_t n;
-    Divisor d1, d2;
+    FastDiv32 d1, d2;
     float v0, v1, v2;
 };
 
@@ -308,9 +286,9 @@ raw_write_kernel(RawOut a, RawWork w, float *__restrict__ xyz,
     const uint32_t limit =
         capacity - base < total ? (uint32_t)(capacity - base) : total;
     // raster position of the first sample: first = (i * d1 + j) * d2 + k
-    const uint32_t ij = quotient_of(first, a.d2);
+    const uint32_t ij = a.d2.div(first);
     const uint32_t k0 = first - ij * a.d2.d;
-    const uint32_t i0 = quotient_of(ij, a.d1);
+    const uint32_t i0 = a.d1.div(ij);
     const uint32_t j0 = ij - i0 * a.d1.d;
     // the non-empty masks to the first lanes, in order
     const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
@@ -486,8 +464,8 @@ int voxg_raw_write(const unsigned dim[3], const float voxel[3],
     if (!xyz_out) return fail(VOXG_EINVAL, "xyz_out is NULL");
     RawOut a;
     a.n = n;
-    a.d1 = divisor(dim[1]);
-    a.d2 = divisor(dim[2]);
+    a.d1 = make_fastdiv32(dim[1]);
+    a.d2 = make_fastdiv32(dim[2]);
     a.v0 = voxel ? voxel[0] : 1.0f;
     a.v1 = voxel ? voxel[1] : 1.0f;
     a.v2 = voxel ? voxel[2] : 1.0f;
