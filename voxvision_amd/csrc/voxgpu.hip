@@ -3557,9 +3557,10 @@ struct RelaxedCapture {
 // A stream of the library's own on the current device (one each, never
 // captured); null: none to be had.
 hipStream_t own_stream() {
-    static std::map<int, hipStream_t> streams;
+    static hipStream_t streams[64];
     int devid = 0;
-    if (hipGetDevice(&devid) != hipSuccess) return nullptr;
+    if (hipGetDevice(&devid) != hipSuccess || devid < 0 || devid >= 64)
+        return nullptr;
     std::lock_guard<std::mutex> g(g_mu);
     hipStream_t &s = streams[devid];
     if (!s && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess)
@@ -3627,12 +3628,12 @@ void make_ball_grid(const voxg_tree *t) {
 // that are edited again after a few queries, would pay for nothing (a commit
 // of an edited 256^3 scene 5.0 -> 6.1 ms, its tree 12.8 -> 20.1 MB).  Measured
 // on scenes of 53^3 to 256^3, it saves 0.03 to 0.1 ns a query, most often 0.08
-// (4 M of radii 0.5 to 8 in a 256^3 one: 525 us without, 178 with), and 1 to 3
-// us a launch, however small; it takes 170 us, most of them the allocation,
-// and 0.28 ns a cell (0.75 ms for 256^3).  In queries of 0.08 ns: a launch
-// counts for 2^15 more than it has, against 2^21 and 7/2 a cell.  A tree that
-// stops right after its grid was made then has lost about as much as it could
-// have gained.
+// (4 M of radii 0.5 to 8 in a 256^3 one: 525 us without, 178 with), and up to
+// 3 us a launch, however small; allocating and filling it takes 170 us for a
+// 64^3 scene and 0.75 ms for a 256^3 one, about 0.28 ns a cell more.  In
+// queries of 0.08 ns: a launch counts for 2^15 more than it has, against 2^21
+// and 7/2 a cell.  A tree that stops right after its grid was made then has
+// lost about as much as it could have gained.
 constexpr uint64_t kBallLaunch = 1u << 15, kBallGridBase = 1u << 21;
 
 ballgrid::Grid ball_grid_for(const voxg_tree *t, size_t n, hipStream_t stream) {
@@ -3818,7 +3819,10 @@ int voxg_tree_upload(const struct vox_node *root, const float voxel[3],
 
 int voxg_tree_release(voxg_tree *t) {
     if (!t) return 0;
-    if (t->balls.made) (void)hipEventDestroy(t->balls.made);
+    if (t->balls.made) {
+        (void)hipEventSynchronize(t->balls.made);
+        (void)hipEventDestroy(t->balls.made);
+    }
     if (t->balls.mem) HIPCHK(hipFree(t->balls.mem));
     if (t->d_mem) HIPCHK(hipFree(t->d_mem));
     delete t;
