@@ -34,23 +34,23 @@ def _dev_f32(x, n=None, cols=None):
 
 def _other(stream):
     """`stream` if it is another one than the current stream, else None."""
-    if stream is None or \
-            stream.cuda_stream == torch.cuda.current_stream().cuda_stream:
+    if stream is None:
+        return None
+    if stream.cuda_stream == torch.cuda.current_stream().cuda_stream:
         return None
     return stream if isinstance(stream, torch.cuda.Stream) else \
         torch.cuda.ExternalStream(stream.cuda_stream)
 
 
 def _hand_over(stream, *tensors):
-    """Before a launch on `stream` (from _other; None: nothing to do) that
-    uses tensors written on, or allocated for, the current stream: the launch
-    waits for the current stream's work so far, and a tensor that is dropped
-    is not handed out again until `stream` is done with it."""
-    if stream is not None:
-        stream.wait_stream(torch.cuda.current_stream())
-        for t in tensors:
-            if t is not None:
-                t.record_stream(stream)
+    """Before a launch on `stream` (from _other) that uses tensors written
+    on, or allocated for, the current stream: the launch waits for the current
+    stream's work so far, and a tensor that is dropped is not handed out again
+    until `stream` is done with it."""
+    stream.wait_stream(torch.cuda.current_stream())
+    for t in tensors:
+        if t is not None:
+            t.record_stream(stream)
 
 
 def _input(x, stream, rows=False):
@@ -211,7 +211,8 @@ def ray_tree_intersection(tree, o, d, want_leaf=False, hit_init=None,
     else:  # hits are written while other rays are read
         rows = [hit[k][:n] for k in range(3)]
         o, d = (x.clone() if _overlap(x, rows) else x for x in (o, d))
-    _hand_over(other, o, d, vox, leaf, hit[0], hit[1], hit[2])
+    if other is not None:
+        _hand_over(other, o, d, vox, leaf, hit[0], hit[1], hit[2])
     check(L.voxg_ray_batch_rows(tree.handle, n, o.data_ptr(), d.data_ptr(),
                                 vox.data_ptr(),
                                 leaf.data_ptr() if want_leaf else None,
@@ -230,7 +231,9 @@ def ray_counts(tree, o, d, stream=None):
     o = _dev_f32(o).reshape(-1, 3).t().contiguous()
     d = _dev_f32(d).reshape(-1, 3).t().contiguous()
     c = _lib.Counts()
-    _hand_over(_other(stream), o, d)
+    other = _other(stream)
+    if other is not None:
+        _hand_over(other, o, d)
     check(L.voxg_ray_batch_count(tree.handle, o.shape[1], o[0].data_ptr(),
                                  o[1].data_ptr(), o[2].data_ptr(),
                                  d[0].data_ptr(), d[1].data_ptr(),
@@ -251,7 +254,8 @@ def tree_ball_collidep(tree, c, r, stream=None):
     if r.shape[0] < n:
         raise ValueError("a radius for every centre")
     out = torch.empty(n, dtype=torch.uint8, device="cuda")
-    _hand_over(other, c, r, out)
+    if other is not None:
+        _hand_over(other, c, r, out)
     check(L.voxg_ball_batch_rows(tree.handle, n, c.data_ptr(), r.data_ptr(),
                                  out.data_ptr(), _stream(stream)),
           "voxg_ball_batch_rows")
@@ -263,7 +267,9 @@ def ball_counts(tree, c, r, stream=None):
     c = _dev_f32(c).reshape(-1, 3).t().contiguous()
     r = _dev_f32(r).reshape(-1).contiguous()
     cnt = _lib.Counts()
-    _hand_over(_other(stream), c, r)
+    other = _other(stream)
+    if other is not None:
+        _hand_over(other, c, r)
     check(L.voxg_ball_batch_count(tree.handle, c.shape[1], c[0].data_ptr(),
                                   c[1].data_ptr(), c[2].data_ptr(),
                                   r.data_ptr(), C.byref(cnt),
@@ -303,7 +309,8 @@ def raw_select(samples, dim, samplesize, lo=None, hi=None, threshold=None,
     cnt = torch.empty(1, dtype=torch.int64, device="cuda")
     st = _stream(stream)
     other = _other(stream)
-    _hand_over(other, work, cnt)
+    if other is not None:
+        _hand_over(other, work, cnt)
     check(L.voxg_raw_count(samples.data_ptr(), d, samplesize, lo, hi,
                            work.data_ptr(), cnt.data_ptr(), st),
           "voxg_raw_count")
@@ -312,7 +319,8 @@ def raw_select(samples, dim, samplesize, lo=None, hi=None, threshold=None,
     m = int(cnt.item())
     xyz = torch.empty((m, 3), dtype=torch.float32, device="cuda")
     if m:
-        _hand_over(other, xyz)
+        if other is not None:
+            _hand_over(other, xyz)
         check(L.voxg_raw_write(d, v, work.data_ptr(), xyz.data_ptr(), m, st),
               "voxg_raw_write")
     return xyz
